@@ -270,7 +270,7 @@ __device__ __forceinline__ bool bulk_cells(const StepArgs& a, int x0, int y, int
 #pragma unroll
     for (int i = 0; i < V; ++i) {
         if constexpr (M == Mode::EXACT64) {
-            collide_exact<L>(f[i], a.tau);
+            collide_exact<L>(f[i], a.tau, a.omega);
         } else {
             const Calc base = collide_shifted<L, Calc, BRINK, kRcp<M>, IO::SX>(f[i], static_cast<Calc>(a.omega),
                                             BRINK ? alpha[i] : Calc(0),
@@ -596,7 +596,7 @@ __device__ __forceinline__ bool near_cell(const StepArgs& a, int x, int y, int z
 
     bool finite = true;
     if constexpr (M == Mode::EXACT64) {
-        collide_exact<L>(f, a.tau);
+        collide_exact<L>(f, a.tau, a.omega);
     } else {
         Calc alpha = Calc(0);
         if (a.alpha) alpha = static_cast<const Calc*>(a.alpha)[e];
@@ -739,7 +739,7 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
 
     bool finite = true;
     if constexpr (M == Mode::EXACT64) {
-        collide_exact<L>(f, a.tau);
+        collide_exact<L>(f, a.tau, a.omega);
     } else if (a.alpha) {
         const Calc alpha = static_cast<const Calc*>(a.alpha)[e];
         finite = finite_calc(collide_shifted<L, Calc, true, kRcp<M>, IO::SX>(f, static_cast<Calc>(a.omega), alpha,

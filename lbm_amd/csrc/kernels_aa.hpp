@@ -75,7 +75,7 @@ template <class L, Mode M>
 __device__ __forceinline__ void aa_collide(const StepArgs& a, int64_t e, typename Io<M, L>::Calc (&f)[L::Q]) {
     using Calc = typename Io<M, L>::Calc;
     if constexpr (M == Mode::EXACT64) {
-        collide_exact<L>(f, a.tau);
+        collide_exact<L>(f, a.tau, a.omega);
     } else if (a.alpha) {
         const Calc alpha = static_cast<const Calc*>(a.alpha)[e];
         collide_shifted<L, Calc, true, kRcp<M>, Io<M, L>::SX>(f, static_cast<Calc>(a.omega), alpha,
