@@ -189,6 +189,14 @@ int make_plan(lbm_domain* d) {
     p.wpairs = pass_ok && o->step2w != nullptr && walled && d->tune_vec == 0 && !p.freeslip && !p.brink &&
                d->n_fluid > 0 && (d->tune_pass == 2 || d->esize == 4) &&
                p.tb_nblocks <= 0x7fffffffLL;
+    // Below about 12 wavefronts' worth of cells per CU a launch lasts as long
+    // as its chain of dependent accesses, and the pass has the longer one: a
+    // march over three planes, and with walls the emit launch before it.
+    // Measured, us per step, single / pass: D3Q19 fp32 cavity 16^3 9.6 / 15.2,
+    // 32^3 10.0 / 14.4, 48^3 11.7 / 16.3, 64^3 17.7 / 17.3, 96^3 37.4 / 32.2;
+    // periodic 16^3 4.5 / 6.7, 48^3 6.7 / 7.8, 64^3 8.9 / 9.1, 96^3 32.3 /
+    // 20.5 (D3Q15, D3Q27 and 16-bit storage cross at the same sizes).
+    p.small_single = d->tune_pass == 0 && static_cast<int64_t>(d->L.xl) * d->L.yl * d->L.zl < 3 * 65536;
     return LBM_OK;
 }
 
@@ -606,7 +614,8 @@ static int run_steps(lbm_domain* d, uint64_t nsteps, EventLog* log) {
         return LBM_OK;
     }
     uint64_t t = 0;
-    if (d->plan.wpairs) {
+    const bool passes = !d->plan.small_single;
+    if (d->plan.wpairs && passes) {
         // the first step after set-up pulls stored boundary values: single
         if (d->materialised && t < nsteps) {
             const StepArgs a = d->args(d->buf[d->cur], d->buf[d->cur ^ 1], 1);
@@ -623,7 +632,7 @@ static int run_steps(lbm_domain* d, uint64_t nsteps, EventLog* log) {
             d->cur ^= 1;
         }
     }
-    if (d->plan.pairs)
+    if (d->plan.pairs && passes)
         for (; t + 2 <= nsteps; t += 2) {
             // (every source is an interior cell, so the flag has no effect here;
             // it is passed as a single step would take it)

@@ -61,6 +61,9 @@ struct StepPlan {
     int wrules;
     int tb_ntx, tb_nty, tb_zc;
     int tb_nxcd;  // L2 domains the blocks are grouped for (1: identity order)
+    // The automatic setting steps this domain singly although a pass applies:
+    // too few cells for a pass to pay (make_plan).
+    bool small_single;
     int64_t tb_nblocks;
 };
 

@@ -185,3 +185,25 @@ def test_cavity_256_pass_equals_single_steps(storage):
         d.close()
     for a, b in zip(out[1], out[2]):
         assert np.array_equal(bits(a), bits(b))
+
+
+@pytest.mark.parametrize("shape", [(12, 12, 12), (64, 64, 47), (64, 64, 48)])
+@pytest.mark.parametrize("periodic", [0, 1])
+def test_automatic_steps_equal_single_steps(shape, periodic):
+    """The automatic setting (single steps on domains below 3 * 2^16 cells,
+    passes from there on: 64 x 64 x 47 and 48 are either side) gives the bits
+    of single steps."""
+    sc = scenario.Scenario("box", *shape) if periodic else scenario.cavity(*shape, lid=(0.05, 0.02, 0.0))
+    out = []
+    for spp in (1, 0):
+        d = capi.Domain(*shape, 0.6, q=19, storage="f32", periodic=(periodic,) * 3)
+        sc.apply(d)
+        d.finalize()
+        d.set_time_blocking(spp)
+        rng = np.random.default_rng(3)
+        d.init_equilibrium(1 + 1e-3 * rng.standard_normal(shape[::-1]), 0.02 * rng.standard_normal(shape[::-1] + (3,)))
+        d.step(7)
+        out.append(d.moments())
+        d.close()
+    for a, b in zip(*out):
+        assert np.array_equal(bits(a), bits(b))
