@@ -207,11 +207,17 @@ typedef struct lbm_adj_desc {
     int plane_x;            /* interior x of the misfit plane (1..xl) */
     const double* target_u; /* yl*zl*3 target velocities of the plane, y fastest (copied) */
     uint64_t nsteps;        /* steps of the forward run */
-    uint64_t checkpoint_every; /* 0: ceil(sqrt(nsteps)) */
+    uint64_t checkpoint_every; /* 0: automatic (see lbm_adj_create) */
 } lbm_adj_desc;
 
 typedef struct lbm_tape lbm_tape;
 
+/* checkpoint_every = 0: a bulk-only domain (periodic along all axes, no
+ * boundary cells) whose record of density and velocity of every cell and
+ * step (16 bytes a cell and step at fp32, 32 at F64S) takes at most a quarter
+ * of the device's memory and half of what is free keeps that record and
+ * recomputes nothing; any other takes ceil(sqrt(nsteps)). Gradients are the
+ * same bits either way. */
 int lbm_adj_create(lbm_domain* d, const lbm_adj_desc* desc, lbm_tape** out);
 int lbm_adj_destroy(lbm_tape* t);
 /* Forward: alpha (xl*yl*zl, x fastest) replaces the domain's porosity when

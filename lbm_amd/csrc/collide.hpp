@@ -274,9 +274,11 @@ __device__ __forceinline__ void acc_axis(Calc& s, Calc v) {
 // Returns base = drho - 1.5 rho u.u of the incoming values: it is NaN or
 // infinite whenever one of them is, which the batched step uses to flag
 // domains that have diverged (callers that do not need it ignore it).
+// mom (or null): receives drho and u of the incoming values, before the
+// porosity and force act on u: all that the adjoint step reads of them.
 template <class L, class Calc, bool BRINK, bool RCP = false, int SX = 0>
 __device__ __forceinline__ Calc collide_shifted(Calc (&g)[L::Q], Calc omega, Calc alpha,
-                                                Calc tgx, Calc tgy, Calc tgz) {
+                                                Calc tgx, Calc tgy, Calc tgz, Calc* mom = nullptr) {
     static_assert(SX == 0 || RCP, "scaled values take the reciprocal form");
     constexpr Calc kS = static_cast<Calc>(static_cast<double>(1u << SX));
     constexpr Calc kInvS = static_cast<Calc>(1.0 / static_cast<double>(1u << SX));
@@ -305,6 +307,12 @@ __device__ __forceinline__ Calc collide_shifted(Calc (&g)[L::Q], Calc omega, Cal
         ux = jx / rho;
         uy = jy / rho;
         uz = jz / rho;
+    }
+    if (mom) {
+        mom[0] = drho;
+        mom[1] = ux;
+        mom[2] = uy;
+        mom[3] = uz;
     }
     if constexpr (BRINK) {
         const Calc s = Calc(1) - alpha;

@@ -93,7 +93,17 @@ struct StepArgs {
     // element index as kind) and body acceleration; alpha == nullptr disables it.
     const void* alpha;
     double g[3];
+    // Kernels built with HIST: 4 Calc values (drho, u) of the incoming
+    // populations per interior cell, x fastest, written here by the step (and
+    // by a two-step pass's second step at hist2).
+    void* hist;
+    void* hist2;
 };
+
+// Interior cell index, x fastest.
+__host__ __device__ inline int64_t cell_index(const FieldLayout& L, int x, int y, int z) {
+    return (x - 1) + static_cast<int64_t>(L.xl) * ((y - 1) + static_cast<int64_t>(L.yl) * (z - 1));
+}
 
 __host__ __device__ inline int64_t cell_elem(const FieldLayout& L, int x, int y, int z) {
     return L.off + x + L.px * y + L.pxy * z;

@@ -38,6 +38,12 @@ struct alignas(sizeof(T) * V) VecT {
     T v[V];
 };
 
+// drho and u of one cell and step (StepArgs::hist).
+template <class Calc>
+struct alignas(16) Mom4 {
+    Calc v[4];
+};
+
 // Streaming (non-temporal) stores for the bulk output: every value written
 // in a step is read once in the next step, long after it would have been
 // evicted, so keeping it in L2 only displaces source lines.
@@ -182,7 +188,7 @@ __device__ __forceinline__ int wrap_if(int v, int l, int per) {
 // from a ghost cell, is NEAR and is masked out before its values are used.
 // V cells (x0 .. x0+V-1, y, z) of one thread. Returns false when a cell it
 // updated read a NaN or infinite value (finite_calc of the collision's base).
-template <class L, Mode M, int V, bool FLAGS, bool BRINK>
+template <class L, Mode M, int V, bool FLAGS, bool BRINK, bool HIST = false>
 __device__ __forceinline__ bool bulk_cells(const StepArgs& a, int x0, int y, int z,
                                            bool* near_lanes = nullptr) {
     using IO = Io<M, L>;
@@ -272,11 +278,15 @@ __device__ __forceinline__ bool bulk_cells(const StepArgs& a, int x0, int y, int
         if constexpr (M == Mode::EXACT64) {
             collide_exact<L>(f[i], a.tau, a.omega);
         } else {
+            Mom4<Calc> mom;
             const Calc base = collide_shifted<L, Calc, BRINK, kRcp<M>, IO::SX>(f[i], static_cast<Calc>(a.omega),
                                             BRINK ? alpha[i] : Calc(0),
                                             static_cast<Calc>(a.tau * a.g[0]),
                                             static_cast<Calc>(a.tau * a.g[1]),
-                                            static_cast<Calc>(a.tau * a.g[2]));
+                                            static_cast<Calc>(a.tau * a.g[2]), HIST ? mom.v : nullptr);
+            if constexpr (HIST) {
+                if (act[i]) static_cast<Mom4<Calc>*>(a.hist)[cell_index(Ly, x0 + i, y, z)] = mom;
+            }
             finite &= !act[i] || finite_calc(base);
         }
     }
@@ -301,7 +311,7 @@ __device__ __forceinline__ bool bulk_cells(const StepArgs& a, int x0, int y, int
     return finite;
 }
 
-template <class L, Mode M, int V, bool FLAGS, bool BRINK>
+template <class L, Mode M, int V, bool FLAGS, bool BRINK, bool HIST = false>
 __global__ void __launch_bounds__(256) k_bulk(StepArgs a, int nbx, int nby) {
     const int b = blockIdx.x;
     const int bx = b % nbx;
@@ -310,7 +320,7 @@ __global__ void __launch_bounds__(256) k_bulk(StepArgs a, int nbx, int nby) {
     const int z = 1 + t / nby;
     const int xv = bx * blockDim.x + threadIdx.x;
     const int y = 1 + by * blockDim.y + threadIdx.y;
-    bulk_cells<L, M, V, FLAGS, BRINK>(a, 1 + xv * V, y, z);
+    bulk_cells<L, M, V, FLAGS, BRINK, HIST>(a, 1 + xv * V, y, z);
 }
 
 // ---------------------------------------------------------------------------

@@ -75,7 +75,77 @@ __device__ __forceinline__ void objective_grad(const AdjArgs& a, int x, int y, i
     });
 }
 
-// mu = (dC/dh)^T lam at the pre-collision state h; returns dJ/dalpha.
+// c_q . (x, y, z), summed in the order x, y, z (zero terms left out: they add
+// +-0 to a finite sum).
+template <class L, int q, class Calc>
+__device__ __forceinline__ Calc dir_dot(Calc x, Calc y, Calc z) {
+    Calc s{};
+    if constexpr (L::cx(q) != 0) s = L::cx(q) > 0 ? x : -x;
+    if constexpr (L::cy(q) != 0) {
+        if constexpr (L::cx(q) == 0)
+            s = L::cy(q) > 0 ? y : -y;
+        else if constexpr (L::cy(q) > 0)
+            s += y;
+        else
+            s -= y;
+    }
+    if constexpr (L::cz(q) != 0) {
+        if constexpr (L::cx(q) == 0 && L::cy(q) == 0)
+            s = L::cz(q) > 0 ? z : -z;
+        else if constexpr (L::cz(q) > 0)
+            s += z;
+        else
+            s -= z;
+    }
+    return s;
+}
+
+// mu = (dC/dh)^T lam, given drho and u of the pre-collision state h; returns
+// dJ/dalpha. Nothing else of h enters, so a run that keeps these four values
+// per cell and step needs no h.
+template <class L, class Calc, bool BRINK>
+__device__ __forceinline__ Calc adjoint_relax(Calc drho, Calc ux, Calc uy, Calc uz, const Calc (&lam)[L::Q],
+                                              Calc (&mu)[L::Q], Calc omega, Calc alpha, Calc tgx, Calc tgy,
+                                              Calc tgz) {
+    const Calc rho = Calc(1) + drho;
+    Calc s = Calc(1), vx = ux, vy = uy, vz = uz;
+    if constexpr (BRINK) {
+        s = Calc(1) - alpha;
+        vx = ux + tgx;
+        vy = uy + tgy;
+        vz = uz + tgz;
+    }
+    const Calc ex = s * vx, ey = s * vy, ez = s * vz;  // equilibrium velocity
+    const Calc uu = ex * ex + ey * ey + ez * ez;
+    Calc P = Calc(0), S = Calc(0), Vx = Calc(0), Vy = Calc(0), Vz = Calc(0);
+    static_for<0, L::Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const Calc lw = lam[q] * static_cast<Calc>(weight<L>(q));
+        const Calc cu = dir_dot<L, q>(ex, ey, ez);
+        P += lw * (Calc(1) + Calc(3) * cu + Calc(4.5) * cu * cu - Calc(1.5) * uu);
+        const Calc k = lw * (Calc(3) + Calc(9) * cu);
+        if constexpr (L::cx(q) != 0) Vx += Calc(L::cx(q)) * k;
+        if constexpr (L::cy(q) != 0) Vy += Calc(L::cy(q)) * k;
+        if constexpr (L::cz(q) != 0) Vz += Calc(L::cz(q)) * k;
+        S += lw;
+    });
+    Vx -= Calc(3) * S * ex;
+    Vy -= Calc(3) * S * ey;
+    Vz -= Calc(3) * S * ez;
+    const Calc base = P - s * (Vx * ux + Vy * uy + Vz * uz);
+    const Calc one_m_omega = Calc(1) - omega;
+    static_for<0, L::Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const Calc vc = dir_dot<L, q>(Vx, Vy, Vz);
+        mu[q] = one_m_omega * lam[q] + omega * (base + s * vc);
+    });
+    if constexpr (BRINK)
+        return -omega * rho * (Vx * vx + Vy * vy + Vz * vz);
+    else
+        return Calc(0);
+}
+
+// The same from the pre-collision state h itself.
 template <class L, class Calc, bool BRINK>
 __device__ __forceinline__ Calc adjoint_collide(const Calc (&h)[L::Q], const Calc (&lam)[L::Q],
                                                 Calc (&mu)[L::Q], Calc omega, Calc alpha, Calc tgx,
@@ -92,42 +162,7 @@ __device__ __forceinline__ Calc adjoint_collide(const Calc (&h)[L::Q], const Cal
         if constexpr (L::cz(q) < 0) jz -= h[q];
     });
     const Calc rho = Calc(1) + drho;
-    const Calc ux = jx / rho, uy = jy / rho, uz = jz / rho;
-    Calc s = Calc(1), vx = ux, vy = uy, vz = uz;
-    if constexpr (BRINK) {
-        s = Calc(1) - alpha;
-        vx = ux + tgx;
-        vy = uy + tgy;
-        vz = uz + tgz;
-    }
-    const Calc ex = s * vx, ey = s * vy, ez = s * vz;  // equilibrium velocity
-    const Calc uu = ex * ex + ey * ey + ez * ez;
-    Calc P = Calc(0), S = Calc(0), Vx = Calc(0), Vy = Calc(0), Vz = Calc(0);
-    static_for<0, L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        const Calc lw = lam[q] * static_cast<Calc>(weight<L>(q));
-        const Calc cu = Calc(L::cx(q)) * ex + Calc(L::cy(q)) * ey + Calc(L::cz(q)) * ez;
-        P += lw * (Calc(1) + Calc(3) * cu + Calc(4.5) * cu * cu - Calc(1.5) * uu);
-        const Calc k = lw * (Calc(3) + Calc(9) * cu);
-        if constexpr (L::cx(q) != 0) Vx += Calc(L::cx(q)) * k;
-        if constexpr (L::cy(q) != 0) Vy += Calc(L::cy(q)) * k;
-        if constexpr (L::cz(q) != 0) Vz += Calc(L::cz(q)) * k;
-        S += lw;
-    });
-    Vx -= Calc(3) * S * ex;
-    Vy -= Calc(3) * S * ey;
-    Vz -= Calc(3) * S * ez;
-    const Calc base = P - s * (Vx * ux + Vy * uy + Vz * uz);
-    const Calc one_m_omega = Calc(1) - omega;
-    static_for<0, L::Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        const Calc vc = Calc(L::cx(q)) * Vx + Calc(L::cy(q)) * Vy + Calc(L::cz(q)) * Vz;
-        mu[q] = one_m_omega * lam[q] + omega * (base + s * vc);
-    });
-    if constexpr (BRINK)
-        return -omega * rho * (Vx * vx + Vy * vy + Vz * vz);
-    else
-        return Calc(0);
+    return adjoint_relax<L, Calc, BRINK>(drho, jx / rho, jy / rho, jz / rho, lam, mu, omega, alpha, tgx, tgy, tgz);
 }
 
 // Backward step of one BULK cell (all Q neighbours fluid).

@@ -95,11 +95,11 @@ __device__ __forceinline__ T* tb_ptr(T* base, uint32_t byte_off) {
 
 template <class L, Mode M, bool BRINK>
 __device__ __forceinline__ void tb_collide(const StepArgs& a, typename Io<M, L>::Calc (&f)[L::Q],
-                                           typename Io<M, L>::Calc alpha) {
+                                           typename Io<M, L>::Calc alpha, typename Io<M, L>::Calc* mom = nullptr) {
     using Calc = typename Io<M, L>::Calc;
     collide_shifted<L, Calc, BRINK, kRcp<M>, Io<M, L>::SX>(f, static_cast<Calc>(a.omega), BRINK ? alpha : Calc(0),
                                              static_cast<Calc>(a.tau * a.g[0]), static_cast<Calc>(a.tau * a.g[1]),
-                                             static_cast<Calc>(a.tau * a.g[2]));
+                                             static_cast<Calc>(a.tau * a.g[2]), mom);
 }
 
 // Logical block of hardware block b when the hardware deals blocks to nxcd
@@ -114,8 +114,9 @@ __device__ __forceinline__ int tb_logical_block(int b, int nb, int nxcd) {
 }
 
 // Logical block = tx + ntx * (ty + nty * chunk); chunk c covers planes
-// 1 + c * zc .. min((c + 1) * zc, zl).
-template <class L, Mode M, bool BRINK>
+// 1 + c * zc .. min((c + 1) * zc, zl). HIST: both steps store drho and u of
+// their tile cells (a.hist, a.hist2).
+template <class L, Mode M, bool BRINK, bool HIST = false>
 __global__ void __launch_bounds__(256) k_bulk2(StepArgs a, int ntx, int nty, int zc, int nxcd) {
     using IO = Io<M, L>;
     using T = typename IO::T;
@@ -198,7 +199,14 @@ __global__ void __launch_bounds__(256) k_bulk2(StepArgs a, int ntx, int nty, int
             });
             Calc al = Calc(0);
             if constexpr (BRINK) al = alpha[(zs3[1] + ys[1] + xs[1]) / TS];
-            tb_collide<L, M, BRINK>(a, f, al);
+            Mom4<Calc> mom;
+            tb_collide<L, M, BRINK>(a, f, al, HIST ? mom.v : nullptr);
+            if constexpr (HIST) {
+                // tile cells of the chunk, each by its own block
+                if (zs >= z0 && zs <= z1 && pi[k] >= 0 && pi[k] < TB_TX && pj[k] >= 0 && pj[k] < TB_TY &&
+                    x0 + pi[k] <= Ly.xl && y0 + pj[k] <= Ly.yl)
+                    static_cast<Mom4<Calc>*>(a.hist)[cell_index(Ly, x0 + pi[k], y0 + pj[k], zs)] = mom;
+            }
             static_for<0, Q>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
                 const T v = IO::template store<q>(f[q]);
@@ -230,7 +238,9 @@ __global__ void __launch_bounds__(256) k_bulk2(StepArgs a, int ntx, int nty, int
                     const uint32_t eb = TS * (static_cast<uint32_t>(Ly.off) + ox) + pz * zo + py * oy;
                     Calc al = Calc(0);
                     if constexpr (BRINK) al = alpha[eb / TS];
-                    tb_collide<L, M, BRINK>(a, f, al);
+                    Mom4<Calc> mom;
+                    tb_collide<L, M, BRINK>(a, f, al, HIST ? mom.v : nullptr);
+                    if constexpr (HIST) static_cast<Mom4<Calc>*>(a.hist2)[cell_index(Ly, ox, oy, zo)] = mom;
                     static_for<0, Q>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
                         store_stream1<T>(tb_ptr(dst + q * plane, eb), IO::template store<q>(f[q]));

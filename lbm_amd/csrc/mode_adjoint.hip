@@ -1,4 +1,5 @@
 // Adjoint, objective and fp64 dual-number (forward-mode) kernels, D3Q15/19/27.
+#include "kernels_adj2.hpp"
 #include "kernels_adjoint.hpp"
 #include "ops_adjoint.hpp"
 #include "ops_impl.hpp"
@@ -47,6 +48,58 @@ struct AdjImpl {
         return hipGetLastError();
     }
 
+    template <int V>
+    static void launch_hist_step(const StepArgs& a, const StepPlan& p, hipStream_t s) {
+        const dim3 grid(static_cast<uint32_t>(p.nblocks_bulk)), block(p.BX, p.BY, 1);
+        if (p.brink)
+            hipLaunchKernelGGL((k_bulk<L, M, V, false, true, true>), grid, block, 0, s, a, p.nbx, p.nby);
+        else
+            hipLaunchKernelGGL((k_bulk<L, M, V, false, false, true>), grid, block, 0, s, a, p.nbx, p.nby);
+    }
+    static hipError_t hist_step(const StepArgs& a, const StepPlan& p, hipStream_t s) {
+        if (p.V == 2)
+            launch_hist_step<2>(a, p, s);
+        else if (p.V == 1)
+            launch_hist_step<1>(a, p, s);
+        else
+            return hipErrorInvalidValue;
+        return hipGetLastError();
+    }
+    static hipError_t hist_backward(const AdjArgs& a, const StepPlan& p, bool brink, hipStream_t s) {
+        const dim3 grid(static_cast<uint32_t>(p.nblocks_bulk)), block(p.BX, p.BY);
+        if (brink)
+            hipLaunchKernelGGL((k_adj_hist<L, M, true>), grid, block, 0, s, a, p.nbx, p.nby);
+        else
+            hipLaunchKernelGGL((k_adj_hist<L, M, false>), grid, block, 0, s, a, p.nbx, p.nby);
+        return hipGetLastError();
+    }
+    static hipError_t hist_step2(const StepArgs& a, const StepPlan& p, hipStream_t s) {
+        if constexpr (M == Mode::F32) {
+            const dim3 grid(static_cast<uint32_t>(p.tb_nblocks));
+            if (p.brink)
+                hipLaunchKernelGGL((k_bulk2<L, M, true, true>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc,
+                                   p.tb_nxcd);
+            else
+                hipLaunchKernelGGL((k_bulk2<L, M, false, true>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc,
+                                   p.tb_nxcd);
+            return hipGetLastError();
+        } else {
+            return hipErrorInvalidValue;
+        }
+    }
+    static hipError_t hist_backward2(const AdjArgs& a, const StepPlan& p, bool brink, hipStream_t s) {
+        if constexpr (M == Mode::F32) {
+            const dim3 grid(static_cast<uint32_t>(p.tb_nblocks));
+            if (brink)
+                hipLaunchKernelGGL((k_adj2<L, true>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc, p.tb_nxcd);
+            else
+                hipLaunchKernelGGL((k_adj2<L, false>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc, p.tb_nxcd);
+            return hipGetLastError();
+        } else {
+            return hipErrorInvalidValue;
+        }
+    }
+
     static AdjOps make() {
         AdjOps o{};
         o.backward_step = &backward_step;
@@ -54,6 +107,10 @@ struct AdjImpl {
         o.objective_dual = &objective_impl<Mode::DUAL64>;
         o.to_dual = &to_dual;
         o.dual_step = &OpsImpl<L, Mode::DUAL64>::template step_impl<1>;
+        o.hist_step = &hist_step;
+        o.hist_step2 = M == Mode::F32 ? &hist_step2 : nullptr;
+        o.hist_backward = &hist_backward;
+        o.hist_backward2 = M == Mode::F32 ? &hist_backward2 : nullptr;
         o.calc_bytes = sizeof(Calc);
         return o;
     }

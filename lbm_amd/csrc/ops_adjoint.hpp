@@ -29,6 +29,10 @@ struct AdjArgs {
     int objective;
     int plane_x;
     const double* target;  // plane misfit: 3 doubles per (y, z), y fastest
+    // recorded runs (k_adj_hist, k_adj2): drho and u of step t, and of step
+    // t - 1, per interior cell (StepArgs::hist)
+    const void* hist;
+    const void* hist2;
 };
 
 struct AdjOps {
@@ -45,6 +49,14 @@ struct AdjOps {
     hipError_t (*to_dual)(const FieldLayout& Ly, const void* src, void* dst, hipStream_t s);
     // one forward step in dual numbers (plan with V = 1)
     hipError_t (*dual_step)(const StepArgs& a, const StepPlan& p, hipStream_t s, EventLog* log);
+    // Recorded runs of bulk-only domains (kernels_adj2.hpp): a forward step
+    // that records drho and u (plan with V = 1 or 2), two in one pass, an
+    // adjoint step from the record, two in one pass. The passes use the
+    // plan's two-step tiles and chunks and are null where not built.
+    hipError_t (*hist_step)(const StepArgs& a, const StepPlan& p, hipStream_t s);
+    hipError_t (*hist_step2)(const StepArgs& a, const StepPlan& p, hipStream_t s);
+    hipError_t (*hist_backward)(const AdjArgs& a, const StepPlan& p, bool brink, hipStream_t s);
+    hipError_t (*hist_backward2)(const AdjArgs& a, const StepPlan& p, bool brink, hipStream_t s);
     size_t calc_bytes;  // bytes of the mode's arithmetic type (mu buffers)
 };
 
