@@ -312,8 +312,10 @@ int lbm_batch_set_config(lbm_batch* b, int kernel, int vec, int bx_policy, int b
  * conditions). Checkpoints every checkpoint_every steps (k); each domain
  * holds N/k + k + 1 field-sized slots on the device. Backward recomputes
  * each segment and steps the adjoint of all domains with one launch per
- * step. checkpoint_every = 0: k = ceil(sqrt(N)) where those slots fit in
- * free device memory, else two levels as lbm_batch_adj_create2 with
+ * step. checkpoint_every = 0: a record of density and velocity of every cell
+ * and step (16 bytes at fp32, 32 at F64S) and no recompute where that takes
+ * at most a quarter of the device's memory and half of what is free; else
+ * k = ceil(sqrt(N)) where those slots fit in free device memory, else two levels as lbm_batch_adj_create2 with
  * k = ceil(N^(2/3)) and sub_every = ceil(sqrt(k)). D3Q19, F32 or F64S,
  * NoSlip / MovingWall / Inflow. */
 typedef struct lbm_batch_tape lbm_batch_tape;
@@ -326,7 +328,8 @@ int lbm_batch_adj_create(lbm_batch* b, uint64_t nsteps, uint64_t checkpoint_ever
  * with one level. */
 int lbm_batch_adj_create2(lbm_batch* b, uint64_t nsteps, uint64_t checkpoint_every, uint64_t sub_every,
                           lbm_batch_tape** out);
-/* out[0] = k, out[1] = k2 (0: one level), out[2] = slots per domain. */
+/* out[0] = k (N for a recorded run), out[1] = k2 (0: one level), out[2] = slots
+ * per domain. */
 int lbm_batch_adj_levels(lbm_batch_tape* t, uint64_t out[3]);
 int lbm_batch_adj_destroy(lbm_batch_tape* t);
 /* J receives one objective value per domain (or NULL); leaves the final state

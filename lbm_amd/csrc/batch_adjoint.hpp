@@ -28,7 +28,15 @@ struct BatchAdjView {
     const uint8_t* lcond;
     const Cond* conds;
     double tau, omega;
-    double* gw;           // 3 doubles per element: dJ/du_wall accumulated per cell
+    const int* near_idx;  // per element: index of a NEAR cell in the domain's list
+    int64_t nb;           // NEAR cells
+    double* gw;           // 3 doubles per NEAR cell: dJ/du_wall accumulated per cell
+    // Recorded runs: the domain's two buffers, and per step hist_stride Calc
+    // values: drho and u of every interior cell, then 1 + the own sum of every
+    // NEAR cell.
+    void* buf[2];
+    void* hist;
+    int64_t hist_stride;
     int tpp;              // 64-cell tiles per z plane
     double rxl;           // 1 / xl
 };
@@ -39,6 +47,9 @@ struct BatchAdjArgs {
     int64_t ntiles;
     int src_slot, dst_slot;                  // recompute step
     int gprev_slot, mu_in_slot, mu_out_slot; // adjoint step
+    int64_t hist_step;                       // recorded step (1 .. T) of hist_forward and hist_backward
+    int parity;                              // hist_forward: buf[parity] -> buf[parity ^ 1]
+    int* status;                             // hist_forward: non-finite flags as BatchArgs::status
     int terminal;
     int materialised;
     int idx32;  // every domain's plane is under 4 GiB (32-bit byte offsets)
@@ -48,7 +59,12 @@ struct BatchAdjArgs {
 struct BatchAdjOps {
     hipError_t (*recompute)(const BatchAdjArgs& a, int grid, hipStream_t s);
     hipError_t (*backward)(const BatchAdjArgs& a, int grid, hipStream_t s);
-    // out[3 d + k] = sum over the elements of domain d of gw (fixed order)
+    // one forward step of every domain that records, one adjoint step from the record
+    hipError_t (*hist_forward)(const BatchAdjArgs& a, int grid, hipStream_t s);
+    hipError_t (*hist_backward)(const BatchAdjArgs& a, int grid, hipStream_t s);
+    // near_idx[element of list entry i] = i
+    hipError_t (*near_index)(const FieldLayout& Ly, const CellCoord* blist, int64_t nb, int* near_idx, hipStream_t s);
+    // out[3 d + k] = sum over the NEAR cells of domain d of gw (fixed order)
     hipError_t (*reduce)(const BatchAdjView* views, int ndom, double* out, hipStream_t s);
 };
 

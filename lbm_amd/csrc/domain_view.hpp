@@ -98,6 +98,11 @@ struct StepArgs {
     // by a two-step pass's second step at hist2).
     void* hist;
     void* hist2;
+    // any_cell built with HIST: index of a NEAR cell in the domain's list per
+    // element, and per list entry 1 + the sum of the cell's own stored values
+    // (Calc), written for cells with moving-wall links.
+    const int* near_idx;
+    void* rho_own;
 };
 
 // Interior cell index, x fastest.

@@ -43,6 +43,8 @@ template <class Calc>
 struct alignas(16) Mom4 {
     Calc v[4];
 };
+template <class Calc>
+using Mom4Raw = Calc __attribute__((ext_vector_type(4)));  // the same as one memory access
 
 // Streaming (non-temporal) stores for the bulk output: every value written
 // in a step is read once in the next step, long after it would have been
@@ -705,7 +707,9 @@ __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B
     });
 }
 
-template <class L, Mode M, bool FS = true, bool B32 = false>
+// HIST records drho and u of the incoming populations, and 1 + the sum of
+// the own values of a cell with moving-wall links (StepArgs::hist, rho_own).
+template <class L, Mode M, bool FS = true, bool B32 = false, bool HIST = false>
 __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z) {
     using IO = Io<M, L>;
     using T = typename IO::T;
@@ -745,7 +749,20 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
         });
     }
     if (k >= KIND_COND0) return true;
-    if (k == KIND_NEAR && !a.materialised) near_rules<L, M, FS, B32>(a, e, x, y, z, f);
+    if (k == KIND_NEAR && !a.materialised) {
+        near_rules<L, M, FS, B32>(a, e, x, y, z, f);
+        if constexpr (HIST) {  // (read by the moving walls' gradient only)
+            const int lc = glob(a.lcond)[e];
+            if (lc == LCOND_MIXED || cond_at(a.conds, lc).kind == BC_MOVINGWALL) {
+                Calc r = Calc(1);
+                static_for<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    r += IO::template to_calc<q>(plane_ref<B32>(src, q, Ly.plane, e));
+                });
+                glob(static_cast<Calc*>(a.rho_own))[glob(a.near_idx)[e]] = r;
+            }
+        }
+    }
 
     bool finite = true;
     if constexpr (M == Mode::EXACT64) {
@@ -757,8 +774,13 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
                                                 static_cast<Calc>(a.tau * a.g[1]),
                                                 static_cast<Calc>(a.tau * a.g[2])));
     } else {
-        finite = finite_calc(collide_shifted<L, Calc, false, kRcp<M>, IO::SX>(f, static_cast<Calc>(a.omega), Calc(0),
-                                                                      Calc(0), Calc(0), Calc(0)));
+        Mom4<Calc> mom;
+        finite = finite_calc(collide_shifted<L, Calc, false, kRcp<M>, IO::SX>(
+            f, static_cast<Calc>(a.omega), Calc(0), Calc(0), Calc(0), Calc(0), HIST ? mom.v : nullptr));
+        if constexpr (HIST) {
+            const Mom4Raw<Calc> m = {mom.v[0], mom.v[1], mom.v[2], mom.v[3]};
+            glob(static_cast<Mom4Raw<Calc>*>(a.hist))[cell_index(Ly, x, y, z)] = m;
+        }
     }
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;

@@ -546,6 +546,136 @@ __device__ __forceinline__ void adj_any_cell(const AdjArgs& a, int x, int y, int
     }
 }
 
+// adj_any_cell from a recorded run (NoSlip, MovingWall and Inflow
+// conditions, no porosity): drho and u of the step come from a.hist, the own
+// sum of a NEAR cell from rho_own, so the only populations read are mu. A NEAR
+// lane finds its links in its mask: bit q of lmask says that the source x -
+// c_q is not fluid, and that cell is also the consumer x + c_k of k = Q-1-q.
+// Where all links share one condition (lcond) its kind is read once, else
+// once per link, instead of the kinds of all 2 Q neighbours and a condition
+// for each that is not fluid. Same operations in the same order as
+// adj_any_cell.
+template <class L, Mode M, bool B32>
+__device__ __forceinline__ void adj_hist_cell(const AdjArgs& a, const uint32_t* lmask, const uint8_t* lcond, int x,
+                                              int y, int z, typename ElemIdx<B32>::type e, bool near,
+                                              const typename Io<M, L>::Calc* rho_own, const int* near_idx,
+                                              double* __restrict__ gw) {
+    using IO = Io<M, L>;
+    using T = typename IO::T;
+    using Calc = typename IO::Calc;
+    using I = typename ElemIdx<B32>::type;
+    static_assert(sizeof(T) == sizeof(Calc), "mu planes are laid out as field planes");
+    constexpr int Q = L::Q;
+    const FieldLayout& Ly = a.L;
+    const Calc* __restrict__ mi = static_cast<const Calc*>(a.mu_in);
+    const bool wraps = (Ly.per[0] && (x == 1 || x == Ly.xl)) || (Ly.per[1] && (y == 1 || y == Ly.yl)) ||
+                       (Ly.per[2] && (z == 1 || z == Ly.zl));
+    auto nb_elem = [&](auto qc, int sgn) -> I {
+        constexpr int q = decltype(qc)::value;
+        if (!wraps)
+            return e + static_cast<I>(sgn * (L::cx(q) + L::cy(q) * Ly.px + L::cz(q) * Ly.pxy));
+        return elem_at<B32>(Ly, wrap_if(x + sgn * L::cx(q), Ly.xl, Ly.per[0]),
+                            wrap_if(y + sgn * L::cy(q), Ly.yl, Ly.per[1]), wrap_if(z + sgn * L::cz(q), Ly.zl, Ly.per[2]));
+    };
+    const Mom4Raw<Calc> m = glob(static_cast<const Mom4Raw<Calc>*>(a.hist))[cell_index(Ly, x, y, z)];
+    uint32_t lm = 0, walls = 0;  // links; links to moving walls
+    int lc = LCOND_MIXED;
+    if (near) {
+        lm = glob(lmask)[e];
+        lc = glob(lcond)[e];
+    }
+    auto coef = [&](auto qc, const GCond& cd) -> Calc {  // d(wall rule)/d(own density)
+        constexpr int q = decltype(qc)::value;
+        const double cu = L::cx(q) * cd.vel[0] + L::cy(q) * cd.vel[1] + L::cz(q) * cd.vel[2];
+        return static_cast<Calc>(6.0 * weight<L>(q) * cu);
+    };
+    Calc lam[Q];
+    if (a.terminal) {
+        const T* __restrict__ gc = static_cast<const T*>(a.gcur);
+        Calc gf[Q];
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            gf[q] = IO::template to_calc<q>(plane_ref<B32>(gc, q, Ly.plane, e));
+        });
+        objective_grad<L, Calc>(a, x, y, z, gf, lam);
+    } else {
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            lam[q] = plane_ref<B32>(mi, q, Ly.plane, nb_elem(qc, 1));
+        });
+    }
+    if (near) {
+        const bool shared = lc != LCOND_MIXED;
+        if (shared) {
+            if (cond_at(a.conds, lc).kind == BC_MOVINGWALL) walls = lm;
+        } else {
+            static_for<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                if (lm & (1u << q)) {
+                    const uint8_t ks = kind_at(a.kind, nb_elem(qc, -1));
+                    if (cond_at(a.conds, ks - KIND_COND0).kind == BC_MOVINGWALL) walls |= 1u << q;
+                }
+            });
+        }
+        if (!a.terminal) {
+            const bool bounce_all = shared && cond_at(a.conds, lc).kind != BC_INFLOW;
+            Calc wall_term = Calc(0);
+            if (bounce_all) {
+                static_for<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    const Calc back = plane_ref<B32>(mi, Q - 1 - q, Ly.plane, e);
+                    lam[q] = pick_bits(((lm >> (Q - 1 - q)) & 1u) != 0, back, lam[q]);
+                });
+                if (walls) {
+                    const GCond& cd = cond_at(a.conds, lc);
+                    static_for<0, Q>([&](auto qc) {
+                        constexpr int q = decltype(qc)::value;
+                        if (walls & (1u << q)) wall_term += plane_ref<B32>(mi, q, Ly.plane, e) * coef(qc, cd);
+                    });
+                }
+            } else {
+                static_for<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    if (lm & (1u << (Q - 1 - q))) {  // consumer x + c_q not fluid
+                        const int kind = cond_at(a.conds, kind_at(a.kind, nb_elem(qc, 1)) - KIND_COND0).kind;
+                        lam[q] = kind == BC_INFLOW ? Calc(0) : plane_ref<B32>(mi, Q - 1 - q, Ly.plane, e);
+                    }
+                    if (walls & (1u << q))
+                        wall_term += plane_ref<B32>(mi, q, Ly.plane, e) *
+                                     coef(qc, cond_at(a.conds, kind_at(a.kind, nb_elem(qc, -1)) - KIND_COND0));
+                });
+            }
+            static_for<0, Q>([&](auto qc) { lam[decltype(qc)::value] += wall_term; });
+        }
+    }
+    Calc mu[Q];
+    adjoint_relax<L, Calc, false>(m[0], m[1], m[2], m[3], lam, mu, static_cast<Calc>(a.omega), Calc(0), Calc(0),
+                                  Calc(0), Calc(0));
+    Calc* __restrict__ mo = static_cast<Calc*>(a.mu_out);
+    static_for<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        plane_ref<B32>(mo, q, Ly.plane, e) = mu[q];
+    });
+    if (walls && !a.materialised) {
+        const int i = glob(near_idx)[e];
+        const Calc ro = glob(rho_own)[i];
+        double gw0 = 0, gw1 = 0, gw2 = 0;
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            if (walls & (1u << q)) {
+                const double f = static_cast<double>(mu[q] * ro) * 6.0 * weight<L>(q);
+                gw0 += f * L::cx(q);
+                gw1 += f * L::cy(q);
+                gw2 += f * L::cz(q);
+            }
+        });
+        Glob<double>* g = glob(gw) + 3 * static_cast<int64_t>(i);
+        g[0] += gw0;
+        g[1] += gw1;
+        g[2] += gw2;
+    }
+}
+
 // Backward step for NEAR cells (listed): gradients per NEAR cell index.
 template <class L, Mode M, bool BRINK>
 __global__ void __launch_bounds__(128) k_adj_near(AdjArgs a) {

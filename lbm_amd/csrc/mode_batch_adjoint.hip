@@ -94,22 +94,103 @@ __global__ void __launch_bounds__(256) k_badj_backward(BatchAdjArgs b) {
         a.tau = v.tau;
         a.omega = v.omega;
         a.objective = OBJ_KINETIC;
-        adj_any_cell<L, M, false, B32>(a, x, y, z, e, k == KIND_NEAR, v.gw + 3 * static_cast<size_t>(e));
+        const bool near = k == KIND_NEAR;
+        adj_any_cell<L, M, false, B32>(a, x, y, z, e, near, v.gw + (near ? 3 * static_cast<int64_t>(v.near_idx[e]) : 0));
     }
 }
 
-// Per-domain sums of the gradient accumulators: block d sums domain d's
-// interior elements with a fixed assignment and a fixed tree, so the result
-// does not depend on scheduling.
+// Step hist_step's record of a domain (wavefront-uniform, as slot).
+template <class Calc>
+__device__ __forceinline__ Calc* record(const BatchAdjView& v, int64_t step) {
+    const uint64_t p = reinterpret_cast<uint64_t>(static_cast<Calc*>(v.hist) + (step - 1) * v.hist_stride);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(p & 0xffffffffu)));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(p >> 32)));
+    return reinterpret_cast<Calc*>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+__device__ __forceinline__ int64_t record_near(const BatchAdjView& v) {
+    return 4 * static_cast<int64_t>(v.L.xl) * v.L.yl * v.L.zl;
+}
+
+// One forward step of every domain, recording.
+template <class L, Mode M, bool B32>
+__global__ void __launch_bounds__(256) k_badj_hist_forward(BatchAdjArgs b) {
+    using Calc = typename StorageOf<M>::Calc;
+    const int lane = threadIdx.x & 63;
+    const TileWalk w = tile_walk(b.ntiles, b.nxcd);
+    for (int t = w.t; t < w.end; t += w.stride) {
+        const TileRef tr = b.tiles[t];
+        const BatchAdjView& v = b.views[tr.dom];
+        int x, y, z;
+        if (!tile_cell(v, tr.local, lane, x, y, z)) continue;
+        StepArgs a{};
+        a.L = v.L;
+        a.src = v.buf[b.parity];
+        a.dst = v.buf[b.parity ^ 1];
+        a.kind = v.kind;
+        a.lmask = v.lmask;
+        a.lcond = v.lcond;
+        a.conds = v.conds;
+        a.materialised = b.materialised;
+        a.tau = v.tau;
+        a.omega = v.omega;
+        Calc* r = record<Calc>(v, b.hist_step);
+        a.hist = r;
+        a.rho_own = r + record_near(v);
+        a.near_idx = v.near_idx;
+        if (!any_cell<L, M, false, B32, true>(a, x, y, z)) b.status[tr.dom] = 1;
+    }
+}
+
+// One adjoint step of every domain from the record of step hist_step: mu in
+// mu_in_slot to mu_out_slot; kinetic-energy objective.
+template <class L, Mode M, bool B32>
+__global__ void __launch_bounds__(256) k_badj_hist_backward(BatchAdjArgs b) {
+    using T = typename StorageOf<M>::T;
+    using Calc = typename StorageOf<M>::Calc;
+    const int lane = threadIdx.x & 63;
+    const TileWalk w = tile_walk(b.ntiles, b.nxcd);
+    for (int t = w.t; t < w.end; t += w.stride) {
+        const TileRef tr = b.tiles[t];
+        const BatchAdjView& v = b.views[tr.dom];
+        int x, y, z;
+        if (!tile_cell(v, tr.local, lane, x, y, z)) continue;
+        const auto e = elem_at<B32>(v.L, x, y, z);
+        const uint8_t k = kind_at(v.kind, e);
+        if (k >= KIND_COND0) continue;
+        AdjArgs a{};
+        a.L = v.L;
+        a.gcur = v.gfinal;
+        a.mu_in = slot<T>(v, b.mu_in_slot);
+        a.mu_out = slot<T>(v, b.mu_out_slot);
+        a.kind = v.kind;
+        a.conds = v.conds;
+        a.materialised = b.materialised;
+        a.terminal = b.terminal;
+        a.tau = v.tau;
+        a.omega = v.omega;
+        a.objective = OBJ_KINETIC;
+        const Calc* r = record<Calc>(v, b.hist_step);
+        a.hist = r;
+        adj_hist_cell<L, M, B32>(a, v.lmask, v.lcond, x, y, z, e, k == KIND_NEAR, r + record_near(v), v.near_idx, v.gw);
+    }
+}
+
+// near_idx[element of NEAR cell i] = i
+__global__ void __launch_bounds__(256) k_badj_near_index(FieldLayout Ly, const CellCoord* blist, int64_t nb, int* near_idx) {
+    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+    if (i >= nb) return;
+    const CellCoord c = blist[i];
+    near_idx[cell_elem(Ly, c.x, c.y, c.z)] = static_cast<int>(i);
+}
+
+// Per-domain sums of the gradient accumulators: block d sums domain d's NEAR
+// cells with a fixed assignment and a fixed tree, so the result does not
+// depend on scheduling.
 __global__ void __launch_bounds__(256) k_badj_reduce(const BatchAdjView* views, double* out) {
     const BatchAdjView& v = views[blockIdx.x];
-    const int64_t n = static_cast<int64_t>(v.L.xl) * v.L.yl * v.L.zl;
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        const int x = 1 + static_cast<int>(i % v.L.xl);
-        const int y = 1 + static_cast<int>((i / v.L.xl) % v.L.yl);
-        const int z = 1 + static_cast<int>(i / (static_cast<int64_t>(v.L.xl) * v.L.yl));
-        const double* g = v.gw + 3 * cell_elem(v.L, x, y, z);
+    for (int64_t i = threadIdx.x; i < v.nb; i += blockDim.x) {
+        const double* g = v.gw + 3 * i;
         s0 += g[0];
         s1 += g[1];
         s2 += g[2];
@@ -143,6 +224,26 @@ struct BatchAdjImpl {
             hipLaunchKernelGGL((k_badj_backward<L, M, false>), dim3(grid), dim3(256), 0, s, a);
         return hipGetLastError();
     }
+    static hipError_t hist_forward(const BatchAdjArgs& a, int grid, hipStream_t s) {
+        if (a.idx32)
+            hipLaunchKernelGGL((k_badj_hist_forward<L, M, true>), dim3(grid), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((k_badj_hist_forward<L, M, false>), dim3(grid), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
+    static hipError_t hist_backward(const BatchAdjArgs& a, int grid, hipStream_t s) {
+        if (a.idx32)
+            hipLaunchKernelGGL((k_badj_hist_backward<L, M, true>), dim3(grid), dim3(256), 0, s, a);
+        else
+            hipLaunchKernelGGL((k_badj_hist_backward<L, M, false>), dim3(grid), dim3(256), 0, s, a);
+        return hipGetLastError();
+    }
+    static hipError_t near_index(const FieldLayout& Ly, const CellCoord* blist, int64_t nb, int* near_idx, hipStream_t s) {
+        if (nb > 0)
+            hipLaunchKernelGGL(k_badj_near_index, dim3(static_cast<uint32_t>((nb + 255) / 256)), dim3(256), 0, s, Ly,
+                               blist, nb, near_idx);
+        return hipGetLastError();
+    }
     static hipError_t reduce(const BatchAdjView* views, int ndom, double* out, hipStream_t s) {
         hipLaunchKernelGGL(k_badj_reduce, dim3(ndom), dim3(256), 0, s, views, out);
         return hipGetLastError();
@@ -151,6 +252,9 @@ struct BatchAdjImpl {
         BatchAdjOps o{};
         o.recompute = &recompute;
         o.backward = &backward;
+        o.hist_forward = &hist_forward;
+        o.hist_backward = &hist_backward;
+        o.near_index = &near_index;
         o.reduce = &reduce;
         return o;
     }
