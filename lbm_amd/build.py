@@ -41,6 +41,7 @@ NOFMA = ["-ffp-contract=off"]
 UNITS = {
     "capi.hip": [],
     "capi_noalloc.hip": [],
+    "capi_fields.hip": [],
     "capi_adjoint.hip": [],
     "mode_adjoint.hip": NOFMA,
     "capi_batch.hip": [],

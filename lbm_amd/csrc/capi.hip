@@ -221,6 +221,10 @@ void free_device(lbm_domain* d) {
     d->d_out4 = nullptr;
 }
 
+}  // namespace
+
+namespace lbm_amd {
+
 int fill_initial(lbm_domain* d, void* buf) {
     // EXACT64 holds the weights; shifted modes hold w - w = 0.
     if (d->mode != Mode::EXACT64) {
@@ -237,7 +241,7 @@ int fill_initial(lbm_domain* d, void* buf) {
     return LBM_OK;
 }
 
-}  // namespace
+}  // namespace lbm_amd
 
 extern "C" {
 
@@ -338,6 +342,7 @@ int lbm_domain_create(const lbm_desc* desc, lbm_domain** out) {
         if (rc) return bail(rc, last_error());
     }
     if (hipStreamSynchronize(d->stream) != hipSuccess) return bail(LBM_ERR_HIP, "initial fill failed");
+    staging_domain_created();
     *out = d;
     return LBM_OK;
 }
@@ -349,6 +354,7 @@ int lbm_domain_destroy(lbm_domain* d) {
     free_device(d);
     if (d->stream) (void)hipStreamDestroy(d->stream);
     delete d;
+    staging_domain_destroyed();
     return LBM_OK;
 }
 
@@ -754,44 +760,6 @@ int lbm_set_pdf(lbm_domain* d, const double* in) {
     if (e != hipSuccess) return fail(LBM_ERR_HIP, std::string("set_pdf: ") + hipGetErrorString(e));
     d->materialised = true;
     d->aa_phase = 0;
-    return LBM_OK;
-}
-
-int lbm_init_equilibrium(lbm_domain* d, const double* rho, const double* u) {
-    if (int rc = check_handle(d)) return rc;
-    if (!d->finalized) return fail(LBM_ERR_STATE, "call lbm_finalize first (fluid cells are needed)");
-    if (!rho || !u) return fail(LBM_ERR_ARG, "null input");
-    const size_t n = static_cast<size_t>(d->L.xl) * d->L.yl * d->L.zl;
-    if (d->aa) {
-        // boundary cells back to the weights, as the two-buffer layout holds them
-        if (int rc = fill_initial(d, d->buf[0])) return rc;
-        d->aa_phase = 0;
-    }
-    double* dev = nullptr;
-    HIPCHK(hipMalloc(&dev, 4 * n * sizeof(double)));
-    hipError_t e = hipMemcpyAsync(dev, rho, n * sizeof(double), hipMemcpyHostToDevice, d->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dev + n, u, 3 * n * sizeof(double), hipMemcpyHostToDevice, d->stream);
-    if (e == hipSuccess) e = d->ops->init_eq(d->L, d->buf[d->cur], d->d_kind, dev, dev + n, d->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(d->stream);
-    (void)hipFree(dev);
-    if (e != hipSuccess) return fail(LBM_ERR_HIP, std::string("init_equilibrium: ") + hipGetErrorString(e));
-    d->materialised = true;
-    return LBM_OK;
-}
-
-int lbm_moments(lbm_domain* d, double* rho, double* u) {
-    if (int rc = check_handle(d)) return rc;
-    if (int rc = aa_settle(d)) return rc;
-    if (int rc = materialise_boundaries(d)) return rc;
-    const size_t n = static_cast<size_t>(d->L.xl) * d->L.yl * d->L.zl;
-    double* dev = nullptr;
-    HIPCHK(hipMalloc(&dev, 4 * n * sizeof(double)));
-    hipError_t e = d->ops->moments(d->L, d->buf[d->cur], dev, dev + n, d->stream);
-    if (e == hipSuccess && rho) e = hipMemcpyAsync(rho, dev, n * sizeof(double), hipMemcpyDeviceToHost, d->stream);
-    if (e == hipSuccess && u) e = hipMemcpyAsync(u, dev + n, 3 * n * sizeof(double), hipMemcpyDeviceToHost, d->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(d->stream);
-    (void)hipFree(dev);
-    if (e != hipSuccess) return fail(LBM_ERR_HIP, std::string("moments: ") + hipGetErrorString(e));
     return LBM_OK;
 }
 

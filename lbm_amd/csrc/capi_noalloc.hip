@@ -57,7 +57,7 @@ int lbm_moments_noalloc(lbm_domain* d, double* rho, double* u) {
     if (int rc = scratch_for(d->desc.device, &dev)) return rc;
     if (int rc = aa_settle(d)) return rc;
     if (int rc = materialise_boundaries(d)) return rc;
-    hipError_t e = d->ops->moments(d->L, d->buf[d->cur], dev, dev + n, d->stream);
+    hipError_t e = d->ops->moments(d->L, d->buf[d->cur], dev, dev + n, 0, static_cast<int64_t>(n), d->stream);
     if (e == hipSuccess && rho) e = hipMemcpyAsync(rho, dev, n * sizeof(double), hipMemcpyDeviceToHost, d->stream);
     if (e == hipSuccess && u) e = hipMemcpyAsync(u, dev + n, 3 * n * sizeof(double), hipMemcpyDeviceToHost, d->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(d->stream);

@@ -218,6 +218,11 @@ inline std::vector<char> alpha_in_layout(const lbm_domain* d, const double* alph
     return a;
 }
 
+// The state every cell of a buffer starts with (defined in capi.hip).
+int fill_initial(lbm_domain* d, void* buf);
+// Domains alive, for the staging pool (defined in capi_fields.hip).
+void staging_domain_created();
+void staging_domain_destroyed();
 // In-place layout: brings the field back to the natural representation if
 // the last step left it swapped (defined in capi.hip).
 int aa_settle(lbm_domain* d);

@@ -73,14 +73,15 @@ __device__ __forceinline__ void load_cell_f64(const FieldLayout& Ly, const void*
 // density() then velocity(density) of interior cells, x fastest
 // (include/io/vtk.hpp:62-73). EXACT64 follows the reference sums; the shifted
 // modes return rho = 1 + sum g and u = sum c g / rho evaluated in double.
+// Cells i0 .. i0 + n - 1; rho and u hold those cells.
 template <class L, Mode M>
-__global__ void k_moments(FieldLayout Ly, const void* src, double* rho, double* u) {
-    const int64_t n = static_cast<int64_t>(Ly.xl) * Ly.yl * Ly.zl;
+__global__ void k_moments(FieldLayout Ly, const void* src, double* rho, double* u, int64_t i0, int64_t n) {
     const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     if (i >= n) return;
-    const int x = 1 + static_cast<int>(i % Ly.xl);
-    const int y = 1 + static_cast<int>((i / Ly.xl) % Ly.yl);
-    const int z = 1 + static_cast<int>(i / (static_cast<int64_t>(Ly.xl) * Ly.yl));
+    const int64_t c = i0 + i;
+    const int x = 1 + static_cast<int>(c % Ly.xl);
+    const int y = 1 + static_cast<int>((c / Ly.xl) % Ly.yl);
+    const int z = 1 + static_cast<int>(c / (static_cast<int64_t>(Ly.xl) * Ly.yl));
     double f[L::Q];
     load_cell_f64<L, M>(Ly, src, cell_elem(Ly, x, y, z), f);
     double r, v[3];
@@ -170,19 +171,20 @@ static __global__ void __launch_bounds__(256) k_sum_partials(const double* parti
         for (int k = 0; k < 4; ++k) out[k] = s[k];
 }
 
-// Interior fluid cells <- feq(rho, u) from x-fastest interior arrays.
+// Interior fluid cells i0 .. i0 + n - 1 <- feq(rho, u); rho and u hold those
+// cells, x fastest.
 template <class L, Mode M>
 __global__ void k_init_eq(FieldLayout Ly, void* dst_, const uint8_t* kind, const double* rho,
-                          const double* u) {
+                          const double* u, int64_t i0, int64_t n) {
     using IO = Io<M, L>;
     using T = typename IO::T;
     using Calc = typename IO::Calc;
-    const int64_t n = static_cast<int64_t>(Ly.xl) * Ly.yl * Ly.zl;
     const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
     if (i >= n) return;
-    const int x = 1 + static_cast<int>(i % Ly.xl);
-    const int y = 1 + static_cast<int>((i / Ly.xl) % Ly.yl);
-    const int z = 1 + static_cast<int>(i / (static_cast<int64_t>(Ly.xl) * Ly.yl));
+    const int64_t c = i0 + i;
+    const int x = 1 + static_cast<int>(c % Ly.xl);
+    const int y = 1 + static_cast<int>((c / Ly.xl) % Ly.yl);
+    const int z = 1 + static_cast<int>(c / (static_cast<int64_t>(Ly.xl) * Ly.yl));
     const int64_t e = cell_elem(Ly, x, y, z);
     if (kind[e] >= KIND_COND0) return;
     T* dst = static_cast<T*>(dst_);

@@ -88,13 +88,14 @@ struct ModeOps {
                           int nz, hipStream_t s);
     hipError_t (*set_pdf)(const FieldLayout& Ly, void* dst, const double* in, int nx, int ny,
                           int nz, hipStream_t s);
-    hipError_t (*moments)(const FieldLayout& Ly, const void* src, double* rho, double* u,
+    // of interior cells i0 .. i0 + n - 1 (x fastest)
+    hipError_t (*moments)(const FieldLayout& Ly, const void* src, double* rho, double* u, int64_t i0, int64_t n,
                           hipStream_t s);
     // partial must hold 4 * nblocks doubles; out 4 doubles.
     hipError_t (*conservation)(const FieldLayout& Ly, const void* src, const uint8_t* kind,
                                double* partial, int nblocks, double* out, hipStream_t s);
     hipError_t (*init_eq)(const FieldLayout& Ly, void* dst, const uint8_t* kind,
-                          const double* rho, const double* u, hipStream_t s);
+                          const double* rho, const double* u, int64_t i0, int64_t n, hipStream_t s);
     hipError_t (*materialise)(const StepArgs& a, int nx, int ny, int nz, hipStream_t s);
     // in-place (AA) layout: one step from representation phase (0: natural,
     // 1: swapped) to the other; and the swapped -> natural conversion

@@ -162,12 +162,11 @@ struct OpsImpl {
                            dim3(bs), 0, s, Ly, dst, in, GhostDims{nx, ny, nz});
         return hipGetLastError();
     }
-    static hipError_t moments(const FieldLayout& Ly, const void* src, double* rho, double* u,
+    static hipError_t moments(const FieldLayout& Ly, const void* src, double* rho, double* u, int64_t i0, int64_t n,
                               hipStream_t s) {
-        const int64_t n = static_cast<int64_t>(Ly.xl) * Ly.yl * Ly.zl;
         const int bs = 256;
         hipLaunchKernelGGL((k_moments<L, M>), dim3(static_cast<uint32_t>((n + bs - 1) / bs)),
-                           dim3(bs), 0, s, Ly, src, rho, u);
+                           dim3(bs), 0, s, Ly, src, rho, u, i0, n);
         return hipGetLastError();
     }
     static hipError_t conservation(const FieldLayout& Ly, const void* src, const uint8_t* kind,
@@ -178,11 +177,10 @@ struct OpsImpl {
         return hipGetLastError();
     }
     static hipError_t init_eq(const FieldLayout& Ly, void* dst, const uint8_t* kind,
-                              const double* rho, const double* u, hipStream_t s) {
-        const int64_t n = static_cast<int64_t>(Ly.xl) * Ly.yl * Ly.zl;
+                              const double* rho, const double* u, int64_t i0, int64_t n, hipStream_t s) {
         const int bs = 256;
         hipLaunchKernelGGL((k_init_eq<L, M>), dim3(static_cast<uint32_t>((n + bs - 1) / bs)),
-                           dim3(bs), 0, s, Ly, dst, kind, rho, u);
+                           dim3(bs), 0, s, Ly, dst, kind, rho, u, i0, n);
         return hipGetLastError();
     }
     static hipError_t materialise(const StepArgs& a, int nx, int ny, int nz, hipStream_t s) {
