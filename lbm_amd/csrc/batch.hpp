@@ -21,6 +21,7 @@ struct BatchView {
     const uint8_t* kind;
     const uint32_t* lmask;
     const uint8_t* lcond;
+    int span32;           // StepArgs::span32
     const Cond* conds;
     double tau, omega;
     int bx_log2;  // row tiles: threads along x per tile = 1 << bx_log2 (of 256)

@@ -26,6 +26,7 @@ struct BatchAdjView {
     const uint8_t* kind;
     const uint32_t* lmask;
     const uint8_t* lcond;
+    int span32;           // StepArgs::span32
     const Cond* conds;
     double tau, omega;
     const int* near_idx;  // per element: index of a NEAR cell in the domain's list

@@ -215,6 +215,7 @@ void free_device(lbm_domain* d) {
     d->d_lmask = nullptr;
     d->d_lcond = nullptr;
     d->d_blist = nullptr;
+    d->d_rlist = nullptr;
     d->d_conds = nullptr;
     d->d_alpha = nullptr;
     d->d_partial = nullptr;
@@ -505,9 +506,9 @@ int lbm_finalize(lbm_domain* d) {
     // of NEAR cells (bit q: the source x - c_q is not fluid) and the
     // condition their links share (LCOND_MIXED where they differ).
     std::vector<uint8_t> kind(static_cast<size_t>(L.plane), KIND_INERT);
-    std::vector<uint32_t> lmask(static_cast<size_t>(L.plane), 0u);
+    std::vector<uint32_t> lmask(static_cast<size_t>(L.plane), LINK_NOT_FLUID);
     std::vector<uint8_t> lcond(static_cast<size_t>(L.plane), LCOND_MIXED);
-    std::vector<CellCoord> blist;
+    std::vector<CellCoord> blist, rlist;
     uint64_t nfluid = 0, nbulk = 0, nonbulk_interior = 0;
     for (int z = 0; z < d->nz; ++z)
         for (int y = 0; y < d->ny; ++y)
@@ -532,14 +533,16 @@ int lbm_finalize(lbm_domain* d) {
                     if (hs != 0) {
                         m |= 1u << q;
                         const int ci = cond_map[hs - 1];
+                        if (uniq[ci].kind != LBM_BC_NOSLIP) m |= LINK_RULES;
                         shared = shared == -1 ? ci : (shared == ci ? ci : -2);
                     }
                 }
+                lmask[e] = m;
                 if (m) {
                     kind[e] = KIND_NEAR;
-                    lmask[e] = m;
                     if (shared >= 0) lcond[e] = static_cast<uint8_t>(shared);
                     blist.push_back(CellCoord{x, y, z, 0});
+                    if (m & LINK_RULES) rlist.push_back(blist.back());
                     ++nonbulk_interior;
                 } else {
                     kind[e] = KIND_BULK;
@@ -559,7 +562,10 @@ int lbm_finalize(lbm_domain* d) {
     HIPCHK(hipMemcpyAsync(d->d_lcond, lcond.data(), lcond.size(), hipMemcpyHostToDevice, d->stream));
     d->nb = static_cast<int64_t>(blist.size());
     if (d->nb) {
+        d->nr = static_cast<int64_t>(rlist.size());
+        blist.insert(blist.end(), rlist.begin(), rlist.end());
         HIPCHK(hipMalloc(&d->d_blist, blist.size() * sizeof(CellCoord)));
+        d->d_rlist = d->d_blist + d->nb;
         HIPCHK(hipMemcpyAsync(d->d_blist, blist.data(), blist.size() * sizeof(CellCoord),
                               hipMemcpyHostToDevice, d->stream));
         d->device_bytes += blist.size() * sizeof(CellCoord);

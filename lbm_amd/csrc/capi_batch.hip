@@ -87,6 +87,7 @@ int configure(lbm_batch* b, int V, int bx_policy, int bpc, int kernel) {
         v.kind = d->d_kind;
         v.lmask = d->d_lmask;
         v.lcond = d->d_lcond;
+        v.span32 = d->field_bytes < (size_t{1} << 32) ? 1 : 0;
         v.conds = d->d_conds;
         v.tau = d->desc.tau;
         v.omega = 1.0 / d->desc.tau;
@@ -670,6 +671,7 @@ int batch_adj_create(lbm_batch* b, uint64_t nsteps, uint64_t k1, uint64_t k2, bo
         v.kind = d->d_kind;
         v.lmask = d->d_lmask;
         v.lcond = d->d_lcond;
+        v.span32 = d->field_bytes < (size_t{1} << 32) ? 1 : 0;
         v.conds = d->d_conds;
         v.tau = d->desc.tau;
         v.omega = 1.0 / d->desc.tau;

@@ -139,10 +139,12 @@ struct lbm_domain {
     void* buf[2] = {nullptr, nullptr};
     int cur = 0;
     uint8_t* d_kind = nullptr;
-    uint32_t* d_lmask = nullptr;  // per element: non-fluid sources of a NEAR cell (bit q)
+    uint32_t* d_lmask = nullptr;  // per element: link word (domain_view.hpp)
     uint8_t* d_lcond = nullptr;   // per element: their shared condition (same allocation, after d_lmask)
     CellCoord* d_blist = nullptr;
     int64_t nb = 0;
+    CellCoord* d_rlist = nullptr;  // NEAR cells with LINK_RULES (after d_blist, same allocation)
+    int64_t nr = 0;
     Cond* d_conds = nullptr;
     int nconds_dev = 0;
     void* d_alpha = nullptr;
@@ -183,6 +185,9 @@ struct lbm_domain {
         a.kind = d_kind;
         a.lmask = d_lmask;
         a.lcond = d_lcond;
+        a.span32 = field_bytes < (size_t{1} << 32) ? 1 : 0;
+        a.rlist = d_rlist;
+        a.nr = nr;
         a.blist = d_blist;
         a.nb = nb;
         a.conds = d_conds;

@@ -28,6 +28,14 @@ enum : uint8_t {
 constexpr int kMaxConds = KIND_INERT - KIND_COND0;  // 252 distinct conditions
 constexpr uint8_t LCOND_MIXED = 0xFF;  // links of a NEAR cell under more than one condition
 
+// Link word of a cell (StepArgs::lmask): bit q < Q set when the cell is fluid
+// and its source x - c_q is not; LINK_RULES when one of those links has a
+// condition other than NoSlip; LINK_NOT_FLUID for every other cell and for
+// padding.
+constexpr uint32_t LINK_BITS = (1u << 27) - 1;
+constexpr uint32_t LINK_RULES = 1u << 30;
+constexpr uint32_t LINK_NOT_FLUID = 1u << 31;
+
 // Boundary-condition kinds, numbered as in include/lbm_hip.h.
 enum : int {
     BC_NOSLIP = 1,
@@ -76,15 +84,17 @@ struct StepArgs {
     const void* src;
     void* dst;
     const uint8_t* kind;
-    // per element: bit q set when the cell is fluid and its source x - c_q is
-    // not (the links a near-boundary cell takes from boundary rules)
-    const uint32_t* lmask;
+    const uint32_t* lmask;  // link word per element
+    int span32;             // a whole buffer is under 4 GiB: 32-bit byte offsets across planes
     // per element: for a NEAR cell, the condition index shared by every link
     // of its mask, or LCOND_MIXED where they differ (edges and corners);
     // may be null (every cell then takes the per-link path)
     const uint8_t* lcond;
     const CellCoord* blist;  // cells of kind NEAR
     int64_t nb;
+    const CellCoord* rlist;  // those with LINK_RULES
+    int emit_all;            // the walled pass's rlist is blist (k_emit_rules)
+    int64_t nr;
     const Cond* conds;
     int materialised;   // 1: non-fluid sources hold values to be read as stored
     double tau;         // relaxation time

@@ -629,17 +629,89 @@ __device__ __forceinline__ bool near_cell(const StepArgs& a, int x, int y, int z
     return finite;
 }
 
+// Element o of base (B32: at byte offset o) in global memory.
+template <bool B32, class T>
+__device__ __forceinline__ PlaneElem<const T>& elem_ref(const T* base, typename ElemIdx<B32>::type o) {
+    using E = PlaneElem<const T>;
+    using EB = std::conditional_t<IsDual<T>::value, const char, Glob<const char>>;
+    if constexpr (B32)
+        return *reinterpret_cast<E*>(reinterpret_cast<EB*>((E*)base) + o);
+    else
+        return ((E*)base)[o];
+}
+
+// f[q] <- the value at source(q) of plane q (byte offset for B32, else element).
+template <class L, Mode M, bool B32, class Source>
+__device__ __forceinline__ void pull_plain(const typename Io<M, L>::T* __restrict__ src, int64_t plane, Source source,
+                                           typename Io<M, L>::Calc (&f)[L::Q]) {
+    static_for<0, L::Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        f[q] = Io<M, L>::template load<q>(elem_ref<B32>(src + q * plane, source(qc)));
+    });
+}
+
+// ---------------------------------------------------------------------------
+// The Q values a fluid cell takes in: the pulls from x - c_q, and for each
+// link q in `links` (NoSlip sources) its own value of the opposite direction,
+// which is what that rule returns. Where a lane of the wavefront has links,
+// each load's address is selected per lane, so bounce-back costs no loads of
+// its own. (Loading all Q own values beside the pulls, as any rule may need
+// them, the 64-cell tiles of small or narrow domains, where nearly every
+// wavefront holds a wall lane, issued 47 loads a tile for 20 wanted. Single
+// steps: 96^3 fp64 cavity 71.3 -> 57.8 us, 256^3 fp16 cavity 276 -> 254 us,
+// 192 x 96 x 96 D3Q27 fp64 sphere channel 239 -> 206 us.) source(q) is the
+// byte offset (B32) or element of x - c_q in its plane, e the element of x.
+// Selected addresses are 32-bit byte offsets from the buffer where it is
+// under 4 GiB (span32), else (FAR) 64-bit.
+template <class L, Mode M, bool B32, bool FAR = true, class Source>
+__device__ __forceinline__ void pull_all(const typename Io<M, L>::T* __restrict__ src, int64_t plane,
+                                         typename ElemIdx<B32>::type e, uint32_t links, int span32, Source source,
+                                         typename Io<M, L>::Calc (&f)[L::Q]) {
+    using IO = Io<M, L>;
+    using T = typename IO::T;
+    constexpr int Q = L::Q;
+    if (!__any(static_cast<int>(links))) {
+        pull_plain<L, M, B32>(src, plane, source, f);
+        return;
+    }
+    if constexpr (B32) {
+        if (!FAR || span32) {
+            const uint32_t plane_bytes = static_cast<uint32_t>(plane) * static_cast<uint32_t>(sizeof(T));
+            static_for<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                // (the empty asm has the multiples recomputed where they are
+                // used: hoisted, they overflow the scalar registers)
+                uint32_t pb = plane_bytes;
+                asm volatile("" : "+s"(pb));
+                const uint32_t from = source(qc) + q * pb;
+                const uint32_t own = e * static_cast<uint32_t>(sizeof(T)) + (Q - 1 - q) * pb;
+                const uint32_t m = 0u - ((links >> q) & 1u);
+                f[q] = IO::template load<q>(elem_ref<true>(src, (own & m) | (from & ~m)));
+            });
+            return;
+        }
+    }
+    if constexpr (FAR || !B32) static_for<0, Q>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        const T* from = (const T*)&elem_ref<B32>(src + q * plane, source(qc));
+        const T* own = src + ((Q - 1 - q) * plane + static_cast<int64_t>(e));
+        using E = PlaneElem<const T>;
+        f[q] = IO::template load<q>(*(E*)(((links >> q) & 1u) ? own : from));
+    });
+}
+
 // ---------------------------------------------------------------------------
 // One interior cell of any kind, for kernels that hand every cell of a region
-// to a thread (the batched cell tiles). Non-fluid cells return at once. Every
-// direction is first pulled plainly (sources wrapped along periodic axes;
-// along a walled axis the source may be a ghost or solid cell); a NEAR cell
-// then replaces the values pulled from non-fluid sources by their boundary
-// values (as near_cell), and all lanes collide and store together. The bits
+// to a thread (the cell tiles). Non-fluid cells return at once. The link word
+// says which directions bounce back (pull_all); a cell with a link of another
+// rule pulls every direction plainly (sources wrapped along periodic axes;
+// along a walled axis the source may be a ghost or solid cell) and then
+// replaces the values pulled from non-fluid sources by their boundary values
+// (as near_cell). All lanes collide and store together. The bits
 // equal those of bulk_cells / near_cell for the same cell. B32 takes the
 // cell's own and plain-pull addresses as 32-bit byte offsets (planes under
 // 4 GiB). Returns false when a fluid cell read a NaN or infinite value.
-// The pulls of a NEAR cell x (element e, ghosted-box coordinates x, y, z)
+// The pulls of a NEAR cell x with LINK_RULES (element e, ghosted-box coordinates x, y, z)
 // from non-fluid sources, f[q] for every link q of its mask, replaced by
 // their boundary values, from x's stored values in a.src (the reference's
 // boundary pass folded into the pull).
@@ -658,7 +730,7 @@ __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B
         constexpr int kk = decltype(kc)::value;
         return IO::template to_calc<kk>(plane_ref<B32>(src, kk, Ly.plane, e));
     };
-    const uint32_t lm = glob(a.lmask)[e];
+    const uint32_t lm = glob(a.lmask)[e] & LINK_BITS;
     if constexpr (M != Mode::EXACT64 && M != Mode::DUAL64) {
         // Every link under one condition (not FreeSlip, whose rule reads
         // other cells): one branch on its kind, then that family's loads go
@@ -680,12 +752,10 @@ __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B
                     });
                 } else if (ck == BC_INFLOW) {
                     static_for<0, Q>([&](auto qc) { put(qc, static_cast<Calc>(cd.geq[decltype(qc)::value])); });
-                } else if (ck == BC_OUTFLOW || ck == BC_PRESSURE) {
+                } else {  // Outflow, Pressure (cells with NoSlip links only do not come here)
                     static_for<0, Q>([&](auto qc) {
                         put(qc, outflow_rule<L, Calc, decltype(qc)::value>(os, finv(qc), cd));
                     });
-                } else {  // NoSlip
-                    static_for<0, Q>([&](auto qc) { put(qc, finv(qc)); });
                 }
                 return;
             }
@@ -718,38 +788,40 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
     constexpr int Q = L::Q;
     const FieldLayout& Ly = a.L;
     const I e = elem_at<B32>(Ly, x, y, z);
-    const uint8_t k = kind_at(a.kind, e);
+    const uint32_t w = glob(a.lmask)[e];
     const T* __restrict__ src = static_cast<const T*>(a.src);
     T* __restrict__ dst = static_cast<T*>(a.dst);
+    if (w & LINK_NOT_FLUID) return true;
 
-    // Pulls are issued before the kind test (sources of any interior cell lie
-    // inside the ghosted box), so the kind lookup adds no round trip; a
-    // non-fluid cell discards them.
+    // A cell with a link of another rule than NoSlip pulls plainly and
+    // patches all its links below; one in its first step pulls stored values.
+    // (Pulls sent ahead of the link word, with the bounced values loaded
+    // afterwards, took 2 to 14 % longer from 64^3 up and no less below.)
+    constexpr I US = B32 ? static_cast<I>(sizeof(T)) : I(1);  // unit of the sources
     Calc f[Q];
     // Away from the faces of periodic axes every source is a fixed element
     // offset c_x + c_y px + c_z pxy away; on those faces the source wraps.
     const bool wraps = (Ly.per[0] && (x == 1 || x == Ly.xl)) || (Ly.per[1] && (y == 1 || y == Ly.yl)) ||
                        (Ly.per[2] && (z == 1 || z == Ly.zl));
+    auto near_src = [&](auto qc) -> I {
+        constexpr int q = decltype(qc)::value;
+        constexpr int cx = L::cx(q), cy = L::cy(q), cz = L::cz(q);
+        const int64_t d = cx + (cy > 0 ? Ly.px : (cy < 0 ? -Ly.px : 0)) + (cz > 0 ? Ly.pxy : (cz < 0 ? -Ly.pxy : 0));
+        return (e - static_cast<I>(d)) * US;
+    };
+    auto wrap_src = [&](auto qc) -> I {
+        constexpr int q = decltype(qc)::value;
+        return elem_at<B32>(Ly, wrap_if(x - L::cx(q), Ly.xl, Ly.per[0]), wrap_if(y - L::cy(q), Ly.yl, Ly.per[1]),
+                            wrap_if(z - L::cz(q), Ly.zl, Ly.per[2])) * US;
+    };
+    const bool rules = (w & LINK_RULES) && !a.materialised;
+    const uint32_t links = (rules || a.materialised) ? 0u : w;
     if (!wraps) {
-        static_for<0, Q>([&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            constexpr int cx = L::cx(q), cy = L::cy(q), cz = L::cz(q);
-            const int64_t d = cx + (cy > 0 ? Ly.px : (cy < 0 ? -Ly.px : 0)) +
-                              (cz > 0 ? Ly.pxy : (cz < 0 ? -Ly.pxy : 0));
-            f[q] = IO::template load<q>(plane_ref<B32>(src, q, Ly.plane, e - static_cast<I>(d)));
-        });
+        pull_all<L, M, B32>(src, Ly.plane, e, links, a.span32, near_src, f);
     } else {
-        static_for<0, Q>([&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            constexpr int cx = L::cx(q), cy = L::cy(q), cz = L::cz(q);
-            const int sx = wrap_if(x - cx, Ly.xl, Ly.per[0]);
-            const int sy = wrap_if(y - cy, Ly.yl, Ly.per[1]);
-            const int sz = wrap_if(z - cz, Ly.zl, Ly.per[2]);
-            f[q] = IO::template load<q>(plane_ref<B32>(src, q, Ly.plane, elem_at<B32>(Ly, sx, sy, sz)));
-        });
+        pull_all<L, M, B32>(src, Ly.plane, e, links, a.span32, wrap_src, f);
     }
-    if (k >= KIND_COND0) return true;
-    if (k == KIND_NEAR && !a.materialised) {
+    if (rules) {
         near_rules<L, M, FS, B32>(a, e, x, y, z, f);
         if constexpr (HIST) {  // (read by the moving walls' gradient only)
             const int lc = glob(a.lcond)[e];
@@ -795,7 +867,8 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
 // spill.
 template <class L, Mode M>
 constexpr int cells_min_blocks() {
-    return (M == Mode::EXACT64 || M == Mode::F64S || M == Mode::DUAL64 || L::Q > 19) ? 1 : 6;
+    if (M == Mode::EXACT64) return L::Q > 19 ? 1 : 4;
+    return (M == Mode::F64S || M == Mode::DUAL64 || L::Q > 19) ? 1 : 6;
 }
 
 // Cell-tile kernel: wavefront w of the grid takes the 64 cells

@@ -581,7 +581,7 @@ __device__ __forceinline__ void adj_hist_cell(const AdjArgs& a, const uint32_t* 
     uint32_t lm = 0, walls = 0;  // links; links to moving walls
     int lc = LCOND_MIXED;
     if (near) {
-        lm = glob(lmask)[e];
+        lm = glob(lmask)[e] & LINK_BITS;
         lc = glob(lcond)[e];
     }
     auto coef = [&](auto qc, const GCond& cd) -> Calc {  // d(wall rule)/d(own density)

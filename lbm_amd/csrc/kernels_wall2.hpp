@@ -7,13 +7,16 @@
 // tile and a chunk of z planes; per plane it does step 1 on the tile and its
 // one-cell ring, passes g1 through LDS, and step 2 on the tile one plane
 // behind. What boundaries add:
-//   - before the pass, k_emit_rules writes into every boundary link (b, q)
-//     the value the reference's boundary pass leaves there
-//     (include/domain.hpp:157-165): the rule of b for direction q, from the
-//     stored values of the fluid cell x = b + c_q. Each link has one such x,
-//     so one thread per near-boundary cell x writes its links. Step 1 then
-//     pulls every value plainly, as the single-step cell kernel does after
-//     patching its pulls with the same rule values;
+//   - a cell whose links are all NoSlip bounces back in step 1 by selecting
+//     each pull's address (pull_all). For the others (LINK_RULES: moving
+//     walls, inflow, outflow and pressure faces) k_emit_rules, before the
+//     pass, writes into every boundary link (b, q) the value the reference's
+//     boundary pass leaves there (include/domain.hpp:157-165): the rule of b
+//     for direction q, from the stored values of the fluid cell x = b + c_q.
+//     Each link has one such x, so one thread per listed cell x writes its
+//     links, and step 1 pulls them plainly. (Where the buffer takes 4 GiB or
+//     more, emit_all, every near-boundary cell goes that way. With all of them
+//     emitted a 256^3 cavity's pass took 711 us, with the lid's 658);
 //   - non-fluid cells (ghost layer, solids) do neither step and send nothing;
 //   - step 2 needs the rule values of x's non-fluid sources b = x - c_k from
 //     x's own step-1 values. No neighbour sends those (b is not fluid), so
@@ -42,7 +45,7 @@ namespace lbm_amd {
 
 __device__ __forceinline__ int wrap_axis(int v, int l, int per) { return per ? wrap1(v, l) : v; }
 
-// One thread per near-boundary cell x (the domain's list): for every
+// One thread per cell x with LINK_RULES (the domain's list): for every
 // direction q whose source b = x - c_q is not fluid, b[q] in src <- the rule
 // value of (b, q) from x's stored values. Reads fluid cells, writes
 // non-fluid cells only. x's Q values are loaded once, every value is
@@ -56,39 +59,13 @@ __global__ void __launch_bounds__(256) k_emit_rules(StepArgs a) {
     using Calc = typename IO::Calc;
     constexpr int Q = L::Q;
     const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i >= a.nb) return;
-    const CellCoord c = a.blist[i];
+    if (i >= a.nr) return;
+    const CellCoord c = a.rlist[i];
     const FieldLayout& Ly = a.L;
     T* __restrict__ buf = static_cast<T*>(a.dst);
     const uint32_t e = elem_at<true>(Ly, c.x, c.y, c.z);
     const uint32_t lm = glob(a.lmask)[e];
-    if (lm == 0) return;
     const int lc = glob(a.lcond)[e];
-    if (lc != LCOND_MIXED && cond_at(a.conds, lc).kind == BC_NOSLIP) {
-        // Every link NoSlip: the rule value of link q is the cell's own value
-        // of direction q-bar, so only the linked directions are read (a cell
-        // on an x wall has Q values in Q different lines, of which the other
-        // kinds' rules need all for the density). An unlinked direction reads
-        // the first linked one's element instead, a line fetched anyway, so
-        // that every load goes out unconditionally ahead of the masked stores.
-        const int q0 = __builtin_ctz(lm);
-        T v[Q];
-        static_for<0, Q>([&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            v[q] = plane_ref<true>(buf, ((lm >> q) & 1u) ? Q - 1 - q : Q - 1 - q0, Ly.plane, e);
-        });
-        static_for<0, Q>([&](auto qc) {
-            constexpr int q = decltype(qc)::value;
-            if (lm & (1u << q)) {
-                const uint32_t se = elem_at<true>(Ly, wrap_if(c.x - L::cx(q), Ly.xl, Ly.per[0]),
-                                                  wrap_if(c.y - L::cy(q), Ly.yl, Ly.per[1]),
-                                                  wrap_if(c.z - L::cz(q), Ly.zl, Ly.per[2]));
-                plane_ref<true>(buf, q, Ly.plane, se) =
-                    IO::template from_calc<q>(IO::template to_calc<Q - 1 - q>(v[q]));
-            }
-        });
-        return;
-    }
     Calc own[Q];
     OwnAcc<L, Calc> acc;
     static_for<0, Q>([&](auto qc) {
@@ -105,18 +82,18 @@ __global__ void __launch_bounds__(256) k_emit_rules(StepArgs a) {
     if (lc != LCOND_MIXED) {
         const GCond& cd = cond_at(a.conds, lc);
         const int ck = cd.kind;
-        if ((RULES & RULE_MOVINGWALL) != 0 && ck == BC_MOVINGWALL) {
+        if (ck == BC_NOSLIP) {  // (listed where emit_all)
+            static_for<0, Q>([&](auto qc) { put(qc, finv(qc)); });
+        } else if (RULES == RULE_MOVINGWALL || ck == BC_MOVINGWALL) {
             static_for<0, Q>([&](auto qc) {
                 put(qc, moving_wall_rule<L, Calc, decltype(qc)::value>(acc.r, finv(qc), cd));
             });
-        } else if ((RULES & RULE_INFLOW) != 0 && ck == BC_INFLOW) {
+        } else if (ck == BC_INFLOW) {
             static_for<0, Q>([&](auto qc) { put(qc, static_cast<Calc>(cd.geq[decltype(qc)::value])); });
-        } else if ((RULES & RULE_OUTFLOW) != 0 && (ck == BC_OUTFLOW || ck == BC_PRESSURE)) {
+        } else {  // Outflow, Pressure
             static_for<0, Q>([&](auto qc) {
                 put(qc, outflow_rule<L, Calc, decltype(qc)::value>(acc.r, finv(qc), cd));
             });
-        } else {  // NoSlip
-            static_for<0, Q>([&](auto qc) { put(qc, finv(qc)); });
         }
     } else {
         static_for<0, Q>([&](auto qc) {
@@ -228,15 +205,15 @@ __global__ void __launch_bounds__(256) k_wall2(StepArgs a, int ntx, int nty, int
             if (k < TB_OUT) wm[k & (TB_OUT - 1)] = 0;
             if (!live[k]) continue;
             const uint32_t e = (zs3[1] + py * static_cast<uint32_t>(gy[k]) + TS * static_cast<uint32_t>(gx[k])) / TS;
-            const uint8_t kd = kind_at(a.kind, e);
-            if (kd >= KIND_COND0) continue;
+            const uint32_t w = glob(a.lmask)[e];
+            if (w & LINK_NOT_FLUID) continue;
             fl[k] = true;
             // a tile cell of the chunk next to non-fluid cells: its links
             uint32_t lm = 0;
             int lc = LCOND_MIXED;
-            if (k < TB_OUT && kd == KIND_NEAR && zs >= z0 && zs <= z1) {
-                lm = glob(a.lmask)[e];
-                lc = glob(a.lcond)[e];
+            if (k < TB_OUT && zs >= z0 && zs <= z1) {
+                lm = w;
+                if (w & LINK_RULES) lc = glob(a.lcond)[e];
             }
             const uint32_t xs[3] = {TS * static_cast<uint32_t>(wrap_axis(gx[k] - 1, Ly.xl, Ly.per[0])),
                                     TS * static_cast<uint32_t>(gx[k]),
@@ -245,12 +222,12 @@ __global__ void __launch_bounds__(256) k_wall2(StepArgs a, int ntx, int nty, int
                                     py * static_cast<uint32_t>(gy[k]),
                                     py * static_cast<uint32_t>(wrap_axis(gy[k] + 1, Ly.yl, Ly.per[1]))};
             Calc f[Q];
-            static_for<0, Q>([&](auto qc) {
+            pull_all<L, M, true, false>(src, plane, e, (a.emit_all || (w & LINK_RULES)) ? 0u : w, 1, [&](auto qc) -> uint32_t {
                 constexpr int q = decltype(qc)::value;
                 // source x - c_q: index 0 for c = +1, 1 for 0, 2 for -1
                 constexpr int ix = 1 - L::cx(q), iy = 1 - L::cy(q), iz = 1 - L::cz(q);
-                f[q] = IO::template load<q>(tb_at(src + q * plane, zs3[iz] + ys[iy] + xs[ix]));
-            });
+                return zs3[iz] + ys[iy] + xs[ix];
+            }, f);
             collide_shifted<L, Calc, false, kRcp<M>, IO::SX>(f, static_cast<Calc>(a.omega), Calc(0), Calc(0), Calc(0),
                                                             Calc(0));
             static_for<0, Q>([&](auto qc) {
@@ -318,6 +295,13 @@ __global__ void __launch_bounds__(256) k_wall2(StepArgs a, int ntx, int nty, int
             const uint32_t lm = wm[k];
             if (!lm) continue;
             const int c = k * 256 + tid;
+            if (!(lm & LINK_RULES)) {  // bounce-back: the opposite direction's value as it is
+                static_for<0, Q>([&](auto qc) {
+                    constexpr int q = decltype(qc)::value;
+                    if (lm & (1u << q)) lds[S::template slot<q>()][c] = hold[k][Q - 1 - q];
+                });
+                continue;
+            }
             OwnAcc<L, Calc> acc;
             static_for<0, Q>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
@@ -336,18 +320,16 @@ __global__ void __launch_bounds__(256) k_wall2(StepArgs a, int ntx, int nty, int
             if (lc != LCOND_MIXED) {
                 const GCond& cd = cond_at(a.conds, lc);
                 const int ck = cd.kind;
-                if ((RULES & RULE_MOVINGWALL) != 0 && ck == BC_MOVINGWALL) {
+                if (RULES == RULE_MOVINGWALL || ck == BC_MOVINGWALL) {
                     static_for<0, Q>([&](auto qc) {
                         put(qc, moving_wall_rule<L, Calc, decltype(qc)::value>(acc.r, finv(qc), cd));
                     });
-                } else if ((RULES & RULE_INFLOW) != 0 && ck == BC_INFLOW) {
+                } else if (ck == BC_INFLOW) {
                     static_for<0, Q>([&](auto qc) { put(qc, static_cast<Calc>(cd.geq[decltype(qc)::value])); });
-                } else if ((RULES & RULE_OUTFLOW) != 0 && (ck == BC_OUTFLOW || ck == BC_PRESSURE)) {
+                } else {  // Outflow, Pressure
                     static_for<0, Q>([&](auto qc) {
                         put(qc, outflow_rule<L, Calc, decltype(qc)::value>(acc.r, finv(qc), cd));
                     });
-                } else {  // NoSlip
-                    static_for<0, Q>([&](auto qc) { put(qc, finv(qc)); });
                 }
             } else {
                 static_for<0, Q>([&](auto qc) {

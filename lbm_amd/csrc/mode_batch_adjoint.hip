@@ -57,6 +57,7 @@ __global__ void __launch_bounds__(256) k_badj_recompute(BatchAdjArgs b) {
         a.kind = v.kind;
         a.lmask = v.lmask;
         a.lcond = v.lcond;
+    a.span32 = v.span32;
         a.conds = v.conds;
         a.materialised = b.materialised;
         a.tau = v.tau;
@@ -129,6 +130,7 @@ __global__ void __launch_bounds__(256) k_badj_hist_forward(BatchAdjArgs b) {
         a.kind = v.kind;
         a.lmask = v.lmask;
         a.lcond = v.lcond;
+    a.span32 = v.span32;
         a.conds = v.conds;
         a.materialised = b.materialised;
         a.tau = v.tau;

@@ -45,7 +45,8 @@ struct OpsImpl {
 
     template <int... Vs>
     static hipError_t step_impl(const StepArgs& a, const StepPlan& p, hipStream_t s, EventLog* log) {
-        if (p.cells) {
+        // (the dual-number run steps in rows)
+        if constexpr (M != Mode::DUAL64) if (p.cells) {
             if (p.freeslip) {
                 if (p.idx32)
                     launch_cells<true, true>(a, p, s);
@@ -101,12 +102,17 @@ struct OpsImpl {
                static_cast<size_t>(TbSlots<L>::NSLOT) * TB_CELLS * sizeof(typename Io<M, L>::T) <= 65536;
     }
     template <int RULES>
-    static void launch_wall2(const StepArgs& a, const StepPlan& p, hipStream_t s) {
-        if (a.nb > 0) {
+    static void launch_wall2(StepArgs a, const StepPlan& p, hipStream_t s) {
+        if (!a.span32) {
+            a.emit_all = 1;
+            a.rlist = a.blist;
+            a.nr = a.nb;
+        }
+        if (a.nr > 0) {
             // boundary links of the source buffer, from its fluid cells
             StepArgs e = a;
             e.dst = const_cast<void*>(a.src);
-            hipLaunchKernelGGL((k_emit_rules<L, M, RULES>), dim3(static_cast<uint32_t>((a.nb + 255) / 256)), dim3(256),
+            hipLaunchKernelGGL((k_emit_rules<L, M, RULES>), dim3(static_cast<uint32_t>((a.nr + 255) / 256)), dim3(256),
                                0, s, e);
         }
         hipLaunchKernelGGL((k_wall2<L, M, RULES>), dim3(static_cast<uint32_t>(p.tb_nblocks)), dim3(256), 0, s, a,

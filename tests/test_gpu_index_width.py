@@ -86,3 +86,29 @@ def test_batch_and_batched_adjoint_same_bits_for_both_index_widths(storage):
         assert np.array_equal(bits(f32), bits(f64))
     assert np.array_equal(bits(out[32][1]), bits(out[64][1]))
     assert np.array_equal(bits(out[32][2]), bits(out[64][2]))
+
+
+def test_buffer_of_4_gib_and_more():
+    """A cavity whose planes are under 4 GiB and whose buffer is not
+    (58.8 M cells, D3Q19 fp32): bounce-back addresses take 64 bits in the cell
+    tiles, and the two-step pass emits the links of every near-boundary cell.
+    Both give the bits of 64-bit element indices."""
+    shape = (1400, 210, 200)
+    d = capi.Domain(*shape, 0.6, q=19, storage="f32")
+    scenario.cavity(*shape, lid=(0.05, 0.02, 0.0)).apply(d)
+    d.finalize()
+    assert d.info()["field_bytes"] >= 1 << 32
+    rng = np.random.default_rng(5)
+    rho, u = 1 + 1e-3 * rng.standard_normal(shape[::-1]), np.zeros(shape[::-1] + (3,))
+    out = []
+    for bits, spp in ((64, 1), (32, 1), (32, 2)):
+        d.set_index_width(bits)
+        d.set_time_blocking(spp)
+        assert d.info()["steps_per_pass"] == spp
+        d.init_equilibrium(rho, u)
+        d.step(5)
+        out.append(d.moments())
+    d.close()
+    for r, v in out[1:]:
+        assert np.array_equal(r, out[0][0]) and np.array_equal(v, out[0][1])
+    assert np.abs(out[0][1]).max() > 1e-3
