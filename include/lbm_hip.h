@@ -354,8 +354,8 @@ typedef struct lbm_info {
     int nconds;                /* distinct boundary conditions */
     int cell_tiles;            /* 1: steps run as 64-cell tiles per wavefront (k_cells) */
     int layout;                /* enum lbm_layout */
-    int steps_per_pass;        /* 2: lbm_step runs pairs of steps as one pass (k_bulk2; the automatic
-                                * setting steps domains of less than 3 * 2^16 cells singly) */
+    int steps_per_pass;        /* 2: lbm_step runs pairs of steps as one pass (the automatic setting
+                                * steps domains below the sizes of lbm_set_time_blocking singly) */
     int z_chunk;               /* planes per block of the two-step pass */
 } lbm_info;
 int lbm_get_info(lbm_domain* d, lbm_info* info);
@@ -386,9 +386,11 @@ int lbm_set_index_width(lbm_domain* d, int bits);
  * in-place layout or a vector width set by lbm_set_tuning steps singly.
  * Results on fluid cells are the same bits as single steps. steps_per_pass:
  * 0 (default, automatic): two steps per pass where that measured faster,
- * which leaves domains with boundary cells in 16-bit storage, and
- * domains of less than 3 * 2^16 cells, stepping singly; 2: two steps per pass wherever it applies; 1: single steps. z_chunk: planes per
- * block of the pass (0 = automatic). No reference counterpart: a scheduling
+ * which leaves domains with boundary cells in 16-bit storage stepping
+ * singly, and domains of few cells: under 3 * 2^16 without boundary cells,
+ * under 600 000 with, under 3 000 000 with solid cells inside the box;
+ * 2: two steps per pass wherever it applies; 1: single steps. z_chunk:
+ * planes per block of the pass (0 = automatic). No reference counterpart: a scheduling
  * choice of this implementation. */
 int lbm_set_time_blocking(lbm_domain* d, int steps_per_pass, int z_chunk);
 

@@ -189,14 +189,23 @@ int make_plan(lbm_domain* d) {
     p.wpairs = pass_ok && o->step2w != nullptr && walled && d->tune_vec == 0 && !p.freeslip && !p.brink &&
                d->n_fluid > 0 && (d->tune_pass == 2 || d->esize == 4) &&
                p.tb_nblocks <= 0x7fffffffLL;
-    // Below about 12 wavefronts' worth of cells per CU a launch lasts as long
-    // as its chain of dependent accesses, and the pass has the longer one: a
-    // march over three planes, and with walls the emit launch before it.
-    // Measured, us per step, single / pass: D3Q19 fp32 cavity 16^3 9.6 / 15.2,
-    // 32^3 10.0 / 14.4, 48^3 11.7 / 16.3, 64^3 17.7 / 17.3, 96^3 37.4 / 32.2;
-    // periodic 16^3 4.5 / 6.7, 48^3 6.7 / 7.8, 64^3 8.9 / 9.1, 96^3 32.3 /
-    // 20.5 (D3Q15, D3Q27 and 16-bit storage cross at the same sizes).
-    p.small_single = d->tune_pass == 0 && static_cast<int64_t>(d->L.xl) * d->L.yl * d->L.zl < 3 * 65536;
+    // Where the automatic setting steps singly although a pass applies.
+    // A small domain's launch lasts as long as its chain of dependent
+    // accesses, and the pass has the longer one: a march over three planes,
+    // and with walls the emit launch before it. With walls the pass also holds
+    // half as many wavefronts as the cell tiles, and where solid cells idle
+    // its lanes and put surfaces into most tiles it pays only on fields well
+    // beyond the caches. Measured, us per step, single / pass, fp32:
+    //   periodic D3Q19: 48^3 6.7 / 7.8, 64^3 8.9 / 9.1, 96^3 32.3 / 20.5
+    //     (D3Q15, D3Q27 and 16-bit storage cross at the same sizes);
+    //   cavity D3Q19: 64^3 16.4 / 18.4, 80^3 26.4 / 30.9, 96^3 36.5 / 32.8,
+    //     192^3 207 / 156; D3Q27: 96^3 50.1 / 52.4, 128^3 94.8 / 81.7;
+    //   channel around spheres (fluid 0.8): D3Q19 192x96x96 60.5 / 72.7,
+    //     256x128x128 171 / 148; D3Q27 91.7 / 120, 258 / 243;
+    //   pipe 208x100x100: D3Q19 63.1 / 86.0, D3Q27 90.9 / 153.
+    const uint64_t cells = static_cast<uint64_t>(d->L.xl) * d->L.yl * d->L.zl;
+    const uint64_t least = !walled ? 3 * 65536 : (d->n_fluid == cells ? 600000 : 3000000);
+    p.small_single = d->tune_pass == 0 && cells < least;
     return LBM_OK;
 }
 

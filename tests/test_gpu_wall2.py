@@ -187,12 +187,12 @@ def test_cavity_256_pass_equals_single_steps(storage):
         assert np.array_equal(bits(a), bits(b))
 
 
-@pytest.mark.parametrize("shape", [(12, 12, 12), (64, 64, 47), (64, 64, 48)])
-@pytest.mark.parametrize("periodic", [0, 1])
+@pytest.mark.parametrize("shape,periodic", [((12, 12, 12), 0), ((12, 12, 12), 1), ((64, 64, 47), 1), ((64, 64, 48), 1),
+                                            ((100, 100, 59), 0), ((100, 100, 60), 0)])
 def test_automatic_steps_equal_single_steps(shape, periodic):
-    """The automatic setting (single steps on domains below 3 * 2^16 cells,
-    passes from there on: 64 x 64 x 47 and 48 are either side) gives the bits
-    of single steps."""
+    """The automatic setting (single steps on small domains, passes from
+    3 * 2^16 periodic or 600 000 walled cells on: sizes either side) gives the
+    bits of single steps."""
     sc = scenario.Scenario("box", *shape) if periodic else scenario.cavity(*shape, lid=(0.05, 0.02, 0.0))
     out = []
     for spp in (1, 0):
