@@ -28,7 +28,7 @@ struct lbm_batch {
     int device = 0;
     int ncu = 0;
     hipStream_t stream = nullptr;
-    int V = 0, bpc = 8, bx_policy = 0;
+    int V = 0, bpc = 0, bx_policy = 0;
     int kernel = BK_CELLS;      // enum BatchKernel
     bool any_compact = false;   // some domain packs its rows: row kernels take V = 1 only
     bool any_freeslip = false;  // some domain has a FreeSlip condition
@@ -245,7 +245,10 @@ int lbm_batch_create(lbm_domain* const* domains, int n, lbm_batch** out) {
     int V0 = ops->vecs[0];
     for (int i = 0; i < 4 && ops->vecs[i]; ++i)
         if (ops->vecs[i] == d0->plan.V) V0 = d0->plan.V;
-    int rc = configure(b, V0, 0, 8, BK_CELLS);
+    // one block per four cell tiles: a persistent grid of 8 blocks per CU took
+    // 103 against 90 us a step on 30 cavities of 16 to 96 cells a side and 348
+    // against 273 us on 64
+    int rc = configure(b, V0, 0, 0, BK_CELLS);
     if (rc) {
         free_lists(b);
         (void)hipFree(b->d_status);
@@ -769,7 +772,7 @@ int lbm_batch_adj_forward(lbm_batch_tape* t, double* J) {
         a.tiles = t->d_tiles;
         a.ntiles = t->ntiles;
         a.idx32 = b->all_idx32 ? 1 : 0;
-        a.nxcd = xcd_count(b->ncu);
+        a.nxcd = 1;  // (as the forward step)
         a.status = b->d_status;
         HIPCHK(hipMemcpyAsync(t->d_views, t->views.data(), sizeof(BatchAdjView) * t->views.size(),
                               hipMemcpyHostToDevice, b->stream));
@@ -829,11 +832,12 @@ int lbm_batch_adj_backward(lbm_batch_tape* t, double* grad_wall) {
     a.tiles = t->d_tiles;
     a.ntiles = t->ntiles;
     a.idx32 = b->all_idx32 ? 1 : 0;
-    // tiles grouped by L2 domain: the recompute and adjoint steps move more
-    // data per cell than the forward step (slots, mu, gradient accumulators);
-    // measured on 512 cavities over 2000 steps, recompute 7.1 against 8.9 s
-    // and adjoint 10.7 against 11.3 s
-    a.nxcd = xcd_count(b->ncu);
+    // tiles grouped by L2 domain for the checkpointed sweep: its recompute and
+    // adjoint steps move more data per cell than the forward step (slots, mu,
+    // gradient accumulators); measured on 512 cavities over 2000 steps,
+    // recompute 7.1 against 8.9 s and adjoint 10.7 against 11.3 s. From a
+    // record the plain walk is faster, 331 against 340 us a step (64 cavities)
+    a.nxcd = t->hist ? 1 : xcd_count(b->ncu);
     const int grid = grid_for(t);
     Events ev(2);
     HIPCHK(ev.create());
