@@ -205,7 +205,9 @@ int make_plan(lbm_domain* d) {
     //   pipe 208x100x100: D3Q19 63.1 / 86.0, D3Q27 90.9 / 153.
     const uint64_t cells = static_cast<uint64_t>(d->L.xl) * d->L.yl * d->L.zl;
     const uint64_t least = !walled ? 3 * 65536 : (d->n_fluid == cells ? 600000 : 3000000);
-    p.small_single = d->tune_pass == 0 && cells < least;
+    // With walls the cell tiles also gain more from output kept in the
+    // memory-side cache (Put::Keep) than the pass does.
+    p.small_single = d->tune_pass == 0 && (cells < least || (walled && fits_cache(2 * d->field_bytes)));
     return LBM_OK;
 }
 

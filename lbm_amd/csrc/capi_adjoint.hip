@@ -349,6 +349,7 @@ int lbm_adj_backward(lbm_tape* t, double dJ, double* grad_alpha, double grad_wal
     a.objective = t->objective;
     a.plane_x = t->plane_x;
     a.target = t->d_target;
+    a.cached = fits_cache(2 * static_cast<size_t>(d->L.plane) * d->Q * t->ops->calc_bytes);
 
     Events ev(3 * t->nck);
     HIPCHK(ev.create());

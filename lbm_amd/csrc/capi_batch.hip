@@ -32,6 +32,7 @@ struct lbm_batch {
     int kernel = BK_CELLS;      // enum BatchKernel
     bool any_compact = false;   // some domain packs its rows: row kernels take V = 1 only
     bool any_freeslip = false;  // some domain has a FreeSlip condition
+    size_t field_bytes = 0;     // one buffer of every domain
     bool all_idx32 = true;      // every domain's plane is under 4 GiB
     int64_t near_cells = 0;     // NEAR cells of all domains
     BatchView* d_views = nullptr;
@@ -165,6 +166,7 @@ hipError_t enqueue(lbm_batch* b, uint64_t nsteps, int parity, int mat) {
     a.nnear = b->nnear;
     a.freeslip = b->any_freeslip ? 1 : 0;
     a.idx32 = b->all_idx32 ? 1 : 0;
+    a.cached = fits_cache(2 * b->field_bytes);
     // the forward step keeps the plain walk: grouping tiles by L2 domain
     // measured slower there (512 cavities of 16-96 cells a side: 2.43
     // against 2.10 ms per step), while it pays in the adjoint's kernels
@@ -226,6 +228,7 @@ int lbm_batch_create(lbm_domain* const* domains, int n, lbm_batch** out) {
     if (b->ncu <= 0) b->ncu = 256;
     for (const lbm_domain* d : b->doms) {
         b->ncells += static_cast<uint64_t>(d->L.xl) * d->L.yl * d->L.zl;
+        b->field_bytes += d->field_bytes;
         b->any_compact |= d->compact;
         b->any_freeslip |= d->plan.freeslip;
         b->all_idx32 &= d->plan.idx32;
@@ -772,6 +775,7 @@ int lbm_batch_adj_forward(lbm_batch_tape* t, double* J) {
         a.tiles = t->d_tiles;
         a.ntiles = t->ntiles;
         a.idx32 = b->all_idx32 ? 1 : 0;
+    a.cached = fits_cache(2 * b->field_bytes);
         a.nxcd = 1;  // (as the forward step)
         a.status = b->d_status;
         HIPCHK(hipMemcpyAsync(t->d_views, t->views.data(), sizeof(BatchAdjView) * t->views.size(),
@@ -832,6 +836,7 @@ int lbm_batch_adj_backward(lbm_batch_tape* t, double* grad_wall) {
     a.tiles = t->d_tiles;
     a.ntiles = t->ntiles;
     a.idx32 = b->all_idx32 ? 1 : 0;
+    a.cached = fits_cache(2 * b->field_bytes);
     // tiles grouped by L2 domain for the checkpointed sweep: its recompute and
     // adjoint steps move more data per cell than the forward step (slots, mu,
     // gradient accumulators); measured on 512 cavities over 2000 steps,

@@ -46,12 +46,24 @@ struct alignas(16) Mom4 {
 template <class Calc>
 using Mom4Raw = Calc __attribute__((ext_vector_type(4)));  // the same as one memory access
 
-// Streaming (non-temporal) stores for the bulk output: every value written
-// in a step is read once in the next step, long after it would have been
-// evicted, so keeping it in L2 only displaces source lines.
-#ifndef LBM_NT_STORE
-#define LBM_NT_STORE 1
-#endif
+// How a step's output is stored.
+//   Stream: non-temporal. On a field beyond the caches every value is read
+//     long after it would have been evicted, so keeping it only displaces
+//     source lines (256^3 fp32 box 0.456 against 0.470 ms a single step).
+//   Where both buffers fit the 256 MiB memory-side cache (StepArgs::cached)
+//   streamed values would leave it and the next step fetch them from HBM:
+//   Keep: plain (cell tiles, whose wavefronts write parts of lines);
+//   Through: agent scope, written on at once, so that the launch does not end
+//     with the L2s' dirty lines (row kernels and passes, whose wavefronts
+//     write whole lines).
+// Measured, us a step, Stream / Keep / Through, buffers together: passes over
+// periodic D3Q19 boxes fp32 80^3 (98 MB) 19.3 / 16.2 / 15.4, 104^3 (218 MB)
+// 32.0 / 23.5 / 22.4, 112^3 (252 MB) 37.9 / 29.4 / 29.7, 120^3 (289 MB) 42.1 /
+// 38.4 / 38.4, fp16 150^3 (337 MB) 51.8 / 52.6 / 52.0; cell tiles on cavities
+// fp32 48^3 (19 MB) 12.1 / 12.7 / 12.8, 64^3 (63 MB) 16.5 / 15.5 / 15.1, 104^3
+// 53.5 / 40.6 / 40.9, fp16 96^3 (71 MB) 30.5 / 24.7 / 26.6, fp64 64^3 (105 MB)
+// 24.7 / 20.9 / 20.5; 30 batched cavities (340 MB) 90 / 105 / 111.
+enum class Put { Stream, Keep, Through };
 
 template <int BYTES>
 struct RawOf;
@@ -68,40 +80,38 @@ struct RawOf<16> { using type = uint32_t __attribute__((ext_vector_type(4))); };
 template <>
 struct RawOf<32> { using type = uint32_t __attribute__((ext_vector_type(8))); };
 
-template <class T, int V>
-__device__ __forceinline__ void store_stream(T* p, const VecT<T, V>& v) {
-#if LBM_NT_STORE
-    using R = typename RawOf<sizeof(T) * V>::type;
-    R r;
-    __builtin_memcpy(&r, &v, sizeof(R));
-    __builtin_nontemporal_store(r, reinterpret_cast<R*>(p));
-#else
-    *reinterpret_cast<VecT<T, V>*>(p) = v;
-#endif
+template <Put P, class T, class Ptr>
+__device__ __forceinline__ void put(Ptr p, const T& v) {
+    using R = typename RawOf<sizeof(T)>::type;
+    if constexpr (P == Put::Stream) {
+        R r;
+        __builtin_memcpy(&r, &v, sizeof(R));
+        if constexpr (std::is_same<Ptr, T*>::value)
+            __builtin_nontemporal_store(r, reinterpret_cast<R*>(p));
+        else
+            __builtin_nontemporal_store(r, reinterpret_cast<__attribute__((address_space(1))) R*>(p));
+    } else if constexpr (P == Put::Through && sizeof(T) <= 8) {
+        using U = std::conditional_t<sizeof(T) == 8, uint64_t, std::conditional_t<sizeof(T) == 4, uint32_t, uint16_t>>;
+        U u;
+        __builtin_memcpy(&u, &v, sizeof(U));
+        __hip_atomic_store((__attribute__((address_space(1))) U*)p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        *p = v;
+    }
 }
 
-template <class T>
-__device__ __forceinline__ void store_stream1(T* p, T v) {
-#if LBM_NT_STORE
-    using R = typename RawOf<sizeof(T)>::type;
-    R r;
-    __builtin_memcpy(&r, &v, sizeof(R));
-    __builtin_nontemporal_store(r, reinterpret_cast<R*>(p));
-#else
-    *p = v;
-#endif
-}
-
-template <class T>
-__device__ __forceinline__ void store_stream1(__attribute__((address_space(1))) T* p, T v) {
-#if LBM_NT_STORE
-    using R = typename RawOf<sizeof(T)>::type;
-    R r;
-    __builtin_memcpy(&r, &v, sizeof(R));
-    __builtin_nontemporal_store(r, reinterpret_cast<__attribute__((address_space(1))) R*>(p));
-#else
-    *p = v;
-#endif
+// body(policy) with the policy for a field that does or does not fit the
+// caches. The empty asm keeps the compiler from merging the two branches'
+// stores into one without the non-temporal hint.
+template <Put Cached, class Body>
+__device__ __forceinline__ void with_put(int cached, Body body) {
+    if (cached) {
+        asm volatile("");
+        body(std::integral_constant<Put, Cached>{});
+        asm volatile("");
+    } else {
+        body(std::integral_constant<Put, Put::Stream>{});
+    }
 }
 
 // Element indices within a plane: 32-bit where a plane holds less than
@@ -296,19 +306,22 @@ __device__ __forceinline__ bool bulk_cells(const StepArgs& a, int x0, int y, int
     bool all = true;
 #pragma unroll
     for (int i = 0; i < V; ++i) all &= act[i];
-    static_for<0, Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        T* __restrict__ out = dst + q * Ly.plane + e0;
-        if (all) {
-            VecT<T, V> o;
+    with_put<Put::Through>(a.cached, [&](auto pc) {
+        constexpr Put P = decltype(pc)::value;
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            T* __restrict__ out = dst + q * Ly.plane + e0;
+            if (all) {
+                VecT<T, V> o;
 #pragma unroll
-            for (int i = 0; i < V; ++i) o.v[i] = IO::template store<q>(f[i][q]);
-            store_stream<T, V>(out, o);
-        } else {
+                for (int i = 0; i < V; ++i) o.v[i] = IO::template store<q>(f[i][q]);
+                put<P>(reinterpret_cast<VecT<T, V>*>(out), o);
+            } else {
 #pragma unroll
-            for (int i = 0; i < V; ++i)
-                if (act[i]) store_stream1<T>(out + i, IO::template store<q>(f[i][q]));
-        }
+                for (int i = 0; i < V; ++i)
+                    if (act[i]) put<P>(out + i, IO::template store<q>(f[i][q]));
+            }
+        });
     });
     return finite;
 }
@@ -779,7 +792,7 @@ __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B
 
 // HIST records drho and u of the incoming populations, and 1 + the sum of
 // the own values of a cell with moving-wall links (StepArgs::hist, rho_own).
-template <class L, Mode M, bool FS = true, bool B32 = false, bool HIST = false>
+template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false, bool HIST = false>
 __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z) {
     using IO = Io<M, L>;
     using T = typename IO::T;
@@ -856,7 +869,7 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
     }
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        store_stream1<T>(&plane_ref<B32>(dst, q, Ly.plane, e), IO::template store<q>(f[q]));
+        put<CACHED ? Put::Keep : Put::Stream, T>(&plane_ref<B32>(dst, q, Ly.plane, e), IO::template store<q>(f[q]));
     });
     return finite;
 }
@@ -871,9 +884,10 @@ constexpr int cells_min_blocks() {
     return (M == Mode::F64S || M == Mode::DUAL64 || L::Q > 19) ? 1 : 6;
 }
 
+// CACHED: the output policy, built in (a branch on it spilled registers).
 // Cell-tile kernel: wavefront w of the grid takes the 64 cells
 // 64 (w mod tpp) .. + 63 (x fastest) of the z plane 1 + w / tpp.
-template <class L, Mode M, bool FS = true, bool B32 = false>
+template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false>
 __global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cells(StepArgs a, int tpp, double rxl) {
     const int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     const int z = 1 + static_cast<int>(w / tpp);
@@ -891,7 +905,7 @@ __global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cells(StepA
         ++y;
         x -= xl;
     }
-    any_cell<L, M, FS, B32>(a, 1 + static_cast<int>(x), 1 + static_cast<int>(y), z);
+    any_cell<L, M, FS, B32, CACHED>(a, 1 + static_cast<int>(x), 1 + static_cast<int>(y), z);
 }
 
 // Near-boundary kernel: one thread per listed NEAR cell.

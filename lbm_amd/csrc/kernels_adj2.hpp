@@ -71,15 +71,17 @@ __global__ void __launch_bounds__(256) k_adj_hist(AdjArgs a, int nbx, int nby) {
         m.v[0], m.v[1], m.v[2], m.v[3], lam, mu, static_cast<Calc>(a.omega), alpha, static_cast<Calc>(a.tau * a.g[0]),
         static_cast<Calc>(a.tau * a.g[1]), static_cast<Calc>(a.tau * a.g[2]));
     Calc* __restrict__ mo = static_cast<Calc*>(a.mu_out);
-    static_for<0, Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        store_stream1<Calc>(mo + q * Ly.plane + e, mu[q]);
+    with_put<Put::Through>(a.cached, [&](auto pc) {
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            put<decltype(pc)::value>(mo + q * Ly.plane + e, mu[q]);
+        });
     });
     if constexpr (BRINK) a.grad_alpha[e] += static_cast<double>(da);
 }
 
 // Steps t (a.hist) and t - 1 (a.hist2). Logical blocks as k_bulk2.
-template <class L, bool BRINK>
+template <class L, bool BRINK, bool CACHED>
 __global__ void __launch_bounds__(256) k_adj2(AdjArgs a, int ntx, int nty, int zc, int nxcd) {
     using S = TbSlots<L>;
     constexpr int Q = L::Q;
@@ -197,7 +199,7 @@ __global__ void __launch_bounds__(256) k_adj2(AdjArgs a, int ntx, int nty, int z
                                                                   tgx, tgy, tgz);
                     static_for<0, Q>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
-                        store_stream1<float>(tb_ptr(mo + q * plane, eb), mu[q]);
+                        put<CACHED ? Put::Through : Put::Stream>(tb_ptr(mo + q * plane, eb), mu[q]);
                     });
                     if constexpr (BRINK) {
                         double* g = a.grad_alpha + eb / 4u;

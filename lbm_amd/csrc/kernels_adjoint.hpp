@@ -652,9 +652,11 @@ __device__ __forceinline__ void adj_hist_cell(const AdjArgs& a, const uint32_t* 
     adjoint_relax<L, Calc, false>(m[0], m[1], m[2], m[3], lam, mu, static_cast<Calc>(a.omega), Calc(0), Calc(0),
                                   Calc(0), Calc(0));
     Calc* __restrict__ mo = static_cast<Calc*>(a.mu_out);
-    static_for<0, Q>([&](auto qc) {
-        constexpr int q = decltype(qc)::value;
-        plane_ref<B32>(mo, q, Ly.plane, e) = mu[q];
+    with_put<Put::Keep>(a.cached, [&](auto pc) {
+        static_for<0, Q>([&](auto qc) {
+            constexpr int q = decltype(qc)::value;
+            put<decltype(pc)::value, Calc>(&plane_ref<B32>(mo, q, Ly.plane, e), mu[q]);
+        });
     });
     if (walls && !a.materialised) {
         const int i = glob(near_idx)[e];

@@ -115,8 +115,9 @@ __device__ __forceinline__ int tb_logical_block(int b, int nb, int nxcd) {
 
 // Logical block = tx + ntx * (ty + nty * chunk); chunk c covers planes
 // 1 + c * zc .. min((c + 1) * zc, zl). HIST: both steps store drho and u of
-// their tile cells (a.hist, a.hist2).
-template <class L, Mode M, bool BRINK, bool HIST = false>
+// their tile cells (a.hist, a.hist2). CACHED: the output policy, built in (as
+// a branch it cost the 16-bit pass 11 %).
+template <class L, Mode M, bool BRINK, bool CACHED, bool HIST = false>
 __global__ void __launch_bounds__(256) k_bulk2(StepArgs a, int ntx, int nty, int zc, int nxcd) {
     using IO = Io<M, L>;
     using T = typename IO::T;
@@ -243,7 +244,7 @@ __global__ void __launch_bounds__(256) k_bulk2(StepArgs a, int ntx, int nty, int
                     if constexpr (HIST) static_cast<Mom4<Calc>*>(a.hist2)[cell_index(Ly, ox, oy, zo)] = mom;
                     static_for<0, Q>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
-                        store_stream1<T>(tb_ptr(dst + q * plane, eb), IO::template store<q>(f[q]));
+                        put<CACHED ? Put::Through : Put::Stream>(tb_ptr(dst + q * plane, eb), IO::template store<q>(f[q]));
                     });
                 }
             }

@@ -265,7 +265,7 @@ __global__ void __launch_bounds__(256) k_wall2(StepArgs a, int ntx, int nty, int
                                                                 Calc(0), Calc(0));
                 static_for<0, Q>([&](auto qc) {
                     constexpr int q = decltype(qc)::value;
-                    store_stream1<T>(tb_ptr(dst + q * plane, eb), IO::template store<q>(f[q]));
+                    put<Put::Stream>(tb_ptr(dst + q * plane, eb), IO::template store<q>(f[q]));
                 });
             }
         }

@@ -73,27 +73,33 @@ struct AdjImpl {
             hipLaunchKernelGGL((k_adj_hist<L, M, false>), grid, block, 0, s, a, p.nbx, p.nby);
         return hipGetLastError();
     }
+    template <bool BRINK, bool CACHED>
+    static void launch_hist_step2(const StepArgs& a, const StepPlan& p, hipStream_t s) {
+        hipLaunchKernelGGL((k_bulk2<L, M, BRINK, CACHED, true>), dim3(static_cast<uint32_t>(p.tb_nblocks)), dim3(256), 0, s,
+                           a, p.tb_ntx, p.tb_nty, p.tb_zc, p.tb_nxcd);
+    }
     static hipError_t hist_step2(const StepArgs& a, const StepPlan& p, hipStream_t s) {
         if constexpr (M == Mode::F32) {
-            const dim3 grid(static_cast<uint32_t>(p.tb_nblocks));
             if (p.brink)
-                hipLaunchKernelGGL((k_bulk2<L, M, true, true>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc,
-                                   p.tb_nxcd);
+                a.cached ? launch_hist_step2<true, true>(a, p, s) : launch_hist_step2<true, false>(a, p, s);
             else
-                hipLaunchKernelGGL((k_bulk2<L, M, false, true>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc,
-                                   p.tb_nxcd);
+                a.cached ? launch_hist_step2<false, true>(a, p, s) : launch_hist_step2<false, false>(a, p, s);
             return hipGetLastError();
         } else {
             return hipErrorInvalidValue;
         }
     }
+    template <bool BRINK, bool CACHED>
+    static void launch_adj2(const AdjArgs& a, const StepPlan& p, hipStream_t s) {
+        hipLaunchKernelGGL((k_adj2<L, BRINK, CACHED>), dim3(static_cast<uint32_t>(p.tb_nblocks)), dim3(256), 0, s, a,
+                           p.tb_ntx, p.tb_nty, p.tb_zc, p.tb_nxcd);
+    }
     static hipError_t hist_backward2(const AdjArgs& a, const StepPlan& p, bool brink, hipStream_t s) {
         if constexpr (M == Mode::F32) {
-            const dim3 grid(static_cast<uint32_t>(p.tb_nblocks));
             if (brink)
-                hipLaunchKernelGGL((k_adj2<L, true>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc, p.tb_nxcd);
+                a.cached ? launch_adj2<true, true>(a, p, s) : launch_adj2<true, false>(a, p, s);
             else
-                hipLaunchKernelGGL((k_adj2<L, false>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc, p.tb_nxcd);
+                a.cached ? launch_adj2<false, true>(a, p, s) : launch_adj2<false, false>(a, p, s);
             return hipGetLastError();
         } else {
             return hipErrorInvalidValue;

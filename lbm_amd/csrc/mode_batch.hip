@@ -6,7 +6,7 @@ namespace lbm_amd {
 
 namespace {
 
-__device__ __forceinline__ StepArgs view_args(const BatchView& v, int parity, int mat) {
+__device__ __forceinline__ StepArgs view_args(const BatchView& v, int parity, int mat, int cached) {
     StepArgs a{};
     a.L = v.L;
     a.src = v.buf[parity];
@@ -15,6 +15,7 @@ __device__ __forceinline__ StepArgs view_args(const BatchView& v, int parity, in
     a.lmask = v.lmask;
     a.lcond = v.lcond;
     a.span32 = v.span32;
+    a.cached = cached;
     a.conds = v.conds;
     a.materialised = mat;
     a.tau = v.tau;
@@ -39,7 +40,7 @@ __global__ void __launch_bounds__(256) k_batch_bulk(BatchArgs b) {
         const int r = tr.local / v.nbx;
         const int by = r % v.nby;
         const int z = 1 + r / v.nby;
-        const StepArgs a = view_args(v, b.parity, b.materialised);
+        const StepArgs a = view_args(v, b.parity, b.materialised, b.cached);
         const int x0 = 1 + ((bx << bxl) + tx) * V, y = 1 + by * by_n + ty;
         bool finite;
         if constexpr (FUSED) {
@@ -61,7 +62,7 @@ __global__ void __launch_bounds__(256) k_batch_bulk(BatchArgs b) {
 // range of the list); each lane takes one cell of its tile.
 // The tile index is wavefront-uniform; readfirstlane states it, so the tile
 // and the domain view are read into scalar registers once per wavefront.
-template <class L, Mode M, bool FS, bool B32>
+template <class L, Mode M, bool FS, bool B32, bool CACHED = false>
 __global__ void __launch_bounds__(256) k_batch_cells(BatchArgs b) {
     const int lane = threadIdx.x & 63;
     const TileWalk w = tile_walk(b.ntiles, b.nxcd);
@@ -81,8 +82,8 @@ __global__ void __launch_bounds__(256) k_batch_cells(BatchArgs b) {
                 ++y;
                 x -= v.L.xl;
             }
-            const StepArgs a = view_args(v, b.parity, b.materialised);
-            if (!any_cell<L, M, FS, B32>(a, 1 + x, 1 + y, z)) b.status[tr.dom] = 1;
+            const StepArgs a = view_args(v, b.parity, b.materialised, b.cached);
+            if (!any_cell<L, M, FS, B32, CACHED>(a, 1 + x, 1 + y, z)) b.status[tr.dom] = 1;
         }
     }
 }
@@ -92,7 +93,7 @@ __global__ void __launch_bounds__(128) k_batch_near(BatchArgs b) {
     for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < b.nnear;
          i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
         const NearRef n = b.near[i];
-        const StepArgs a = view_args(b.views[n.dom], b.parity, b.materialised);
+        const StepArgs a = view_args(b.views[n.dom], b.parity, b.materialised, b.cached);
         if (!near_cell<L, M>(a, n.x, n.y, n.z)) b.status[n.dom] = 1;
     }
 }
@@ -118,7 +119,9 @@ struct BatchImpl {
                     else
                         hipLaunchKernelGGL((k_batch_cells<L, M, true, false>), dim3(grid_bulk), dim3(256), 0, s, a);
                 } else {
-                    if (a.idx32)
+                    if (a.idx32 && a.cached)
+                        hipLaunchKernelGGL((k_batch_cells<L, M, false, true, true>), dim3(grid_bulk), dim3(256), 0, s, a);
+                    else if (a.idx32)
                         hipLaunchKernelGGL((k_batch_cells<L, M, false, true>), dim3(grid_bulk), dim3(256), 0, s, a);
                     else
                         hipLaunchKernelGGL((k_batch_cells<L, M, false, false>), dim3(grid_bulk), dim3(256), 0, s, a);

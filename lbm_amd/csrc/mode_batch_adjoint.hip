@@ -58,6 +58,7 @@ __global__ void __launch_bounds__(256) k_badj_recompute(BatchAdjArgs b) {
         a.lmask = v.lmask;
         a.lcond = v.lcond;
     a.span32 = v.span32;
+        a.cached = b.cached;
         a.conds = v.conds;
         a.materialised = b.materialised;
         a.tau = v.tau;
@@ -113,7 +114,7 @@ __device__ __forceinline__ int64_t record_near(const BatchAdjView& v) {
 }
 
 // One forward step of every domain, recording.
-template <class L, Mode M, bool B32>
+template <class L, Mode M, bool B32, bool CACHED>
 __global__ void __launch_bounds__(256) k_badj_hist_forward(BatchAdjArgs b) {
     using Calc = typename StorageOf<M>::Calc;
     const int lane = threadIdx.x & 63;
@@ -131,6 +132,7 @@ __global__ void __launch_bounds__(256) k_badj_hist_forward(BatchAdjArgs b) {
         a.lmask = v.lmask;
         a.lcond = v.lcond;
     a.span32 = v.span32;
+        a.cached = b.cached;
         a.conds = v.conds;
         a.materialised = b.materialised;
         a.tau = v.tau;
@@ -139,7 +141,7 @@ __global__ void __launch_bounds__(256) k_badj_hist_forward(BatchAdjArgs b) {
         a.hist = r;
         a.rho_own = r + record_near(v);
         a.near_idx = v.near_idx;
-        if (!any_cell<L, M, false, B32, true>(a, x, y, z)) b.status[tr.dom] = 1;
+        if (!any_cell<L, M, false, B32, CACHED, true>(a, x, y, z)) b.status[tr.dom] = 1;
     }
 }
 
@@ -173,6 +175,7 @@ __global__ void __launch_bounds__(256) k_badj_hist_backward(BatchAdjArgs b) {
         a.objective = OBJ_KINETIC;
         const Calc* r = record<Calc>(v, b.hist_step);
         a.hist = r;
+        a.cached = b.cached;
         adj_hist_cell<L, M, B32>(a, v.lmask, v.lcond, x, y, z, e, k == KIND_NEAR, r + record_near(v), v.near_idx, v.gw);
     }
 }
@@ -227,10 +230,12 @@ struct BatchAdjImpl {
         return hipGetLastError();
     }
     static hipError_t hist_forward(const BatchAdjArgs& a, int grid, hipStream_t s) {
-        if (a.idx32)
-            hipLaunchKernelGGL((k_badj_hist_forward<L, M, true>), dim3(grid), dim3(256), 0, s, a);
+        if (a.idx32 && a.cached)
+            hipLaunchKernelGGL((k_badj_hist_forward<L, M, true, true>), dim3(grid), dim3(256), 0, s, a);
+        else if (a.idx32)
+            hipLaunchKernelGGL((k_badj_hist_forward<L, M, true, false>), dim3(grid), dim3(256), 0, s, a);
         else
-            hipLaunchKernelGGL((k_badj_hist_forward<L, M, false>), dim3(grid), dim3(256), 0, s, a);
+            hipLaunchKernelGGL((k_badj_hist_forward<L, M, false, false>), dim3(grid), dim3(256), 0, s, a);
         return hipGetLastError();
     }
     static hipError_t hist_backward(const BatchAdjArgs& a, int grid, hipStream_t s) {

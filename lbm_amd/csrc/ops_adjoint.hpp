@@ -33,6 +33,7 @@ struct AdjArgs {
     // t - 1, per interior cell (StepArgs::hist)
     const void* hist;
     const void* hist2;
+    int cached;  // StepArgs::cached, for the mu buffers
 };
 
 struct AdjOps {

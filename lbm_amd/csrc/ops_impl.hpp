@@ -37,9 +37,9 @@ struct OpsImpl {
         return true;
     }
 
-    template <bool FS, bool B32>
+    template <bool FS, bool B32, bool CACHED = false>
     static void launch_cells(const StepArgs& a, const StepPlan& p, hipStream_t s) {
-        hipLaunchKernelGGL((k_cells<L, M, FS, B32>), dim3(static_cast<uint32_t>(p.nblocks_cells)), dim3(256), 0, s,
+        hipLaunchKernelGGL((k_cells<L, M, FS, B32, CACHED>), dim3(static_cast<uint32_t>(p.nblocks_cells)), dim3(256), 0, s,
                            a, p.tpp, p.rxl);
     }
 
@@ -54,7 +54,7 @@ struct OpsImpl {
                     launch_cells<true, false>(a, p, s);
             } else {
                 if (p.idx32)
-                    launch_cells<false, true>(a, p, s);
+                    a.cached ? launch_cells<false, true, true>(a, p, s) : launch_cells<false, true>(a, p, s);
                 else
                     launch_cells<false, false>(a, p, s);
             }
@@ -79,15 +79,17 @@ struct OpsImpl {
     static constexpr bool tb_built() {
         return (M == Mode::F32 || M == Mode::F16 || M == Mode::BF16) && tb_lds_bytes<L, M>() <= 65536;
     }
+    template <bool BRINK, bool CACHED>
+    static void launch_step2(const StepArgs& a, const StepPlan& p, hipStream_t s) {
+        hipLaunchKernelGGL((k_bulk2<L, M, BRINK, CACHED>), dim3(static_cast<uint32_t>(p.tb_nblocks)), dim3(256), 0, s, a,
+                           p.tb_ntx, p.tb_nty, p.tb_zc, p.tb_nxcd);
+    }
     static hipError_t step2_impl(const StepArgs& a, const StepPlan& p, hipStream_t s, EventLog* log) {
         if constexpr (tb_built()) {
-            const dim3 grid(static_cast<uint32_t>(p.tb_nblocks));
             if (p.brink)
-                hipLaunchKernelGGL((k_bulk2<L, M, true>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc,
-                                   p.tb_nxcd);
+                a.cached ? launch_step2<true, true>(a, p, s) : launch_step2<true, false>(a, p, s);
             else
-                hipLaunchKernelGGL((k_bulk2<L, M, false>), grid, dim3(256), 0, s, a, p.tb_ntx, p.tb_nty, p.tb_zc,
-                                   p.tb_nxcd);
+                a.cached ? launch_step2<false, true>(a, p, s) : launch_step2<false, false>(a, p, s);
             if (log) log->mark(s, 0);
             return hipGetLastError();
         } else {
@@ -144,9 +146,9 @@ struct OpsImpl {
         int n = 0;
         if constexpr (tb_built()) {
             const hipError_t e = brink ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                                             &n, reinterpret_cast<const void*>(&k_bulk2<L, M, true>), 256, 0)
+                                             &n, reinterpret_cast<const void*>(&k_bulk2<L, M, true, false>), 256, 0)
                                        : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                                             &n, reinterpret_cast<const void*>(&k_bulk2<L, M, false>), 256, 0);
+                                             &n, reinterpret_cast<const void*>(&k_bulk2<L, M, false, false>), 256, 0);
             if (e != hipSuccess) n = 0;
         }
         return n;
