@@ -124,6 +124,10 @@ int make_plan(lbm_domain* d) {
     p.freeslip = false;
     for (const HostCond& c : d->conds) p.freeslip |= c.kind == LBM_BC_FREESLIP;
     p.idx32 = !d->force64 && d->L.plane * static_cast<int64_t>(d->esize) < (int64_t{1} << 32);
+    // Row tiles where rows are padded (x = 1 on a line) and at least half a
+    // wavefront long, from where on their tiles are at least half full; a
+    // launch's y extent, at most 65535, counts the planes.
+    p.tpr = (p.idx32 && !d->compact && d->L.zl <= 65535 && d->L.xl >= 32) ? (d->L.xl + 63) / 64 : 0;
     p.cells = d->tune_vec == 0 && (d->nb > 0 || d->compact) &&
               p.nblocks_cells <= 0x7fffffffLL && (plane_cells + 63) / 64 <= 0x7fffffffLL;
     if (!p.cells && d->compact && V > 1)

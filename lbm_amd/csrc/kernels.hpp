@@ -653,6 +653,51 @@ __device__ __forceinline__ PlaneElem<const T>& elem_ref(const T* base, typename 
         return ((E*)base)[o];
 }
 
+// Byte offsets of a cell's neighbours in a plane under 4 GiB, for a wavefront
+// whose lanes share y and z (row tiles): per lane along x, in scalar registers
+// along y and z, wrapped along periodic axes. Index 0, 1, 2: -1, 0, +1. An
+// access is then a scalar base, direction plane and row included, plus one of
+// three lane offsets: no address arithmetic per lane and no divergence at
+// periodic faces.
+template <class T>
+struct RowNb {
+    uint32_t x[3];
+    int64_t y[3], z[3];
+    __device__ __forceinline__ RowNb(const FieldLayout& L, int cx, int cy, int cz) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            x[i] = static_cast<uint32_t>(sizeof(T)) * static_cast<uint32_t>(wrap_if(cx + i - 1, L.xl, L.per[0]));
+            y[i] = static_cast<int64_t>(sizeof(T)) * L.px * wrap_if(cy + i - 1, L.yl, L.per[1]);
+            z[i] = static_cast<int64_t>(sizeof(T)) * (L.off + L.pxy * wrap_if(cz + i - 1, L.zl, L.per[2]));
+        }
+    }
+    // value of plane q at x + S c_q
+    template <class L, int q, int S>
+    __device__ __forceinline__ Glob<T>& at(T* base, int64_t plane) const {
+        auto* p = reinterpret_cast<Glob<char>*>((Glob<T>*)(base + q * plane)) + (y[1 + S * L::cy(q)] + z[1 + S * L::cz(q)]);
+        return *reinterpret_cast<Glob<T>*>(p + x[1 + S * L::cx(q)]);
+    }
+    template <class L, int q, int S>
+    __device__ __forceinline__ Glob<const T>& at(const T* base, int64_t plane) const {
+        return at<L, q, S>(const_cast<T*>(base), plane);
+    }
+    // the same as an offset from the plane's start
+    template <class L, int q, int S>
+    __device__ __forceinline__ uint32_t offset() const {
+        return x[1 + S * L::cx(q)] + static_cast<uint32_t>(y[1 + S * L::cy(q)] + z[1 + S * L::cz(q)]);
+    }
+};
+
+// Row tiles: wavefront w of z plane 1 + blockIdx.y takes cells 64 (w mod tpr)
+// + 1 .. of row 1 + w / tpr. False past the row or the plane.
+__device__ __forceinline__ bool row_tile_cell(const FieldLayout& L, int tpr, int& x, int& y, int& z) {
+    const int w = static_cast<int>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+    y = 1 + w / tpr;
+    z = 1 + static_cast<int>(blockIdx.y);
+    x = 1 + (w % tpr) * 64 + static_cast<int>(threadIdx.x & 63);
+    return y <= L.yl && x <= L.xl;
+}
+
 // f[q] <- the value at source(q) of plane q (byte offset for B32, else element).
 template <class L, Mode M, bool B32, class Source>
 __device__ __forceinline__ void pull_plain(const typename Io<M, L>::T* __restrict__ src, int64_t plane, Source source,
@@ -676,15 +721,15 @@ __device__ __forceinline__ void pull_plain(const typename Io<M, L>::T* __restric
 // byte offset (B32) or element of x - c_q in its plane, e the element of x.
 // Selected addresses are 32-bit byte offsets from the buffer where it is
 // under 4 GiB (span32), else (FAR) 64-bit.
-template <class L, Mode M, bool B32, bool FAR = true, class Source>
+template <class L, Mode M, bool B32, bool FAR = true, class Source, class Plain>
 __device__ __forceinline__ void pull_all(const typename Io<M, L>::T* __restrict__ src, int64_t plane,
                                          typename ElemIdx<B32>::type e, uint32_t links, int span32, Source source,
-                                         typename Io<M, L>::Calc (&f)[L::Q]) {
+                                         typename Io<M, L>::Calc (&f)[L::Q], Plain plain) {
     using IO = Io<M, L>;
     using T = typename IO::T;
     constexpr int Q = L::Q;
     if (!__any(static_cast<int>(links))) {
-        pull_plain<L, M, B32>(src, plane, source, f);
+        plain();
         return;
     }
     if constexpr (B32) {
@@ -711,6 +756,14 @@ __device__ __forceinline__ void pull_all(const typename Io<M, L>::T* __restrict_
         using E = PlaneElem<const T>;
         f[q] = IO::template load<q>(*(E*)(((links >> q) & 1u) ? own : from));
     });
+}
+
+template <class L, Mode M, bool B32, bool FAR = true, class Source>
+__device__ __forceinline__ void pull_all(const typename Io<M, L>::T* __restrict__ src, int64_t plane,
+                                         typename ElemIdx<B32>::type e, uint32_t links, int span32, Source source,
+                                         typename Io<M, L>::Calc (&f)[L::Q]) {
+    pull_all<L, M, B32, FAR>(src, plane, e, links, span32, source, f,
+                             [&] { pull_plain<L, M, B32>(src, plane, source, f); });
 }
 
 // ---------------------------------------------------------------------------
@@ -792,7 +845,7 @@ __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B
 
 // HIST records drho and u of the incoming populations, and 1 + the sum of
 // the own values of a cell with moving-wall links (StepArgs::hist, rho_own).
-template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false, bool HIST = false>
+template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false, bool HIST = false, bool ROW = false>
 __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z) {
     using IO = Io<M, L>;
     using T = typename IO::T;
@@ -829,7 +882,17 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
     };
     const bool rules = (w & LINK_RULES) && !a.materialised;
     const uint32_t links = (rules || a.materialised) ? 0u : w;
-    if (!wraps) {
+    if constexpr (ROW) {
+        static_assert(B32, "row tiles take 32-bit offsets");
+        const RowNb<T> nb(Ly, x, y, z);
+        pull_all<L, M, true>(src, Ly.plane, e, links, a.span32,
+                             [&](auto qc) { return nb.template offset<L, decltype(qc)::value, -1>(); }, f, [&] {
+            static_for<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                f[q] = IO::template load<q>(nb.template at<L, q, -1>(src, Ly.plane));
+            });
+        });
+    } else if (!wraps) {
         pull_all<L, M, B32>(src, Ly.plane, e, links, a.span32, near_src, f);
     } else {
         pull_all<L, M, B32>(src, Ly.plane, e, links, a.span32, wrap_src, f);
@@ -884,9 +947,21 @@ constexpr int cells_min_blocks() {
     return (M == Mode::F64S || M == Mode::DUAL64 || L::Q > 19) ? 1 : 6;
 }
 
+// Cell-tile kernels. k_cell_rows (planes under 4 GiB, no FreeSlip): row tiles,
+// for padded rows: whole lines per access, y and z in scalar registers, no
+// division per lane. Plane / row tiles, us a
+// single step of a cavity x * 90 * 80: fp32 x 65 25.1 / 22.0, 100 31.3 / 27.4,
+// 250 75.2 / 58.2; fp16 100 22.1 / 22.1, 250 36.9 / 31.7; fp64 40 24.0 / 23.5,
+// 131 74.4 / 62.6, 250 136 / 113 (30, half a tile: 20.8 / 22.0).
+// k_cells: wavefront w of the grid takes the 64 cells 64 (w mod tpp) .. + 63
+// (x fastest) of the z plane 1 + w / tpp, for packed rows and the rest.
 // CACHED: the output policy, built in (a branch on it spilled registers).
-// Cell-tile kernel: wavefront w of the grid takes the 64 cells
-// 64 (w mod tpp) .. + 63 (x fastest) of the z plane 1 + w / tpp.
+template <class L, Mode M, bool CACHED>
+__global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cell_rows(StepArgs a, int tpr) {
+    int x, y, z;
+    if (row_tile_cell(a.L, tpr, x, y, z)) any_cell<L, M, false, true, CACHED, false, true>(a, x, y, z);
+}
+
 template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false>
 __global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cells(StepArgs a, int tpp, double rxl) {
     const int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);

@@ -34,7 +34,6 @@
 
 namespace lbm_amd {
 
-
 // Element of the neighbour x + sgn c_q (wrapped along periodic axes).
 template <class L, int q, class I>
 __device__ __forceinline__ I aa_nb(const FieldLayout& Ly, bool wraps, I e, int x, int y, int z, int sgn) {
@@ -99,30 +98,62 @@ __device__ __forceinline__ void aa_own(const typename Io<M, L>::Calc (&f)[L::Q],
     });
 }
 
-template <class L, Mode M, bool B32>
-__global__ void __launch_bounds__(256) k_aa_eo(StepArgs a, int tpp, double rxl) {
+// Element of the cell's neighbours and accesses relative to it, in either
+// tiling: Nb::at<q, S>() is M[q][x + S c_q], Nb::elem<q, S>() its element.
+template <class L, class T, bool B32>
+struct AaPlane {
+    T* m;
+    const FieldLayout& Ly;
+    int x, y, z;
+    bool wraps;
+    typename ElemIdx<B32>::type e;
+    __device__ __forceinline__ AaPlane(T* m_, const FieldLayout& L_, int x_, int y_, int z_)
+        : m(m_), Ly(L_), x(x_), y(y_), z(z_), wraps(aa_wraps(L_, x_, y_, z_)),
+          e(static_cast<typename ElemIdx<B32>::type>(cell_elem(L_, x_, y_, z_))) {}
+    template <int q, int S>
+    __device__ __forceinline__ auto elem() const {
+        return S == 0 ? e : aa_nb<L, q>(Ly, wraps, e, x, y, z, S);
+    }
+    // M[p][x + S c_q]
+    template <int p, int q, int S>
+    __device__ __forceinline__ Glob<T>& at() const {
+        return plane_ref<B32>(m, p, Ly.plane, elem<q, S>());
+    }
+};
+template <class L, class T>
+struct AaRow {
+    T* m;
+    const FieldLayout& Ly;
+    RowNb<T> nb;
+    uint32_t e;
+    __device__ __forceinline__ AaRow(T* m_, const FieldLayout& L_, int x, int y, int z)
+        : m(m_), Ly(L_), nb(L_, x, y, z), e(elem_at<true>(L_, x, y, z)) {}
+    template <int q, int S>
+    __device__ __forceinline__ uint32_t elem() const {
+        return nb.template offset<L, q, S>() / static_cast<uint32_t>(sizeof(T));
+    }
+    template <int p, int q, int S>
+    __device__ __forceinline__ Glob<T>& at() const {
+        return nb.template at<L, q, S>(m + (p - q) * Ly.plane, Ly.plane);
+    }
+};
+
+template <class L, Mode M, class Nb>
+__device__ __forceinline__ void aa_eo_cell(const StepArgs& a, const Nb& nb) {
     using IO = Io<M, L>;
-    using T = typename IO::T;
     using Calc = typename IO::Calc;
     constexpr int Q = L::Q;
-    const FieldLayout& Ly = a.L;
-    int x, y, z;
-    if (!aa_tile_cell(Ly, tpp, rxl, x, y, z)) return;
-    using I = typename ElemIdx<B32>::type;
-    const I e = static_cast<I>(cell_elem(Ly, x, y, z));
-    const uint8_t k = kind_at(a.kind, e);
+    const uint8_t k = kind_at(a.kind, nb.e);
     if (k >= KIND_COND0) return;
-    T* __restrict__ m = static_cast<T*>(a.dst);
-    const bool wraps = aa_wraps(Ly, x, y, z);
     Calc f[Q];
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        f[q] = IO::template load<q>(plane_ref<B32>(m, q, Ly.plane, aa_nb<L, q>(Ly, wraps, e, x, y, z, -1)));
+        f[q] = IO::template load<q>(nb.template at<q, q, -1>());
     });
-    aa_collide<L, M>(a, static_cast<int64_t>(e), f);
+    aa_collide<L, M>(a, static_cast<int64_t>(nb.e), f);
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        plane_ref<B32>(m, Q - 1 - q, Ly.plane, aa_nb<L, q>(Ly, wraps, e, x, y, z, 1)) = IO::template store<q>(f[q]);
+        nb.template at<Q - 1 - q, q, 1>() = IO::template store<q>(f[q]);
     });
     if (k == KIND_NEAR) {
         Calc own[Q];
@@ -131,51 +162,73 @@ __global__ void __launch_bounds__(256) k_aa_eo(StepArgs a, int tpp, double rxl) 
         static_for<0, Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
             constexpr int j = Q - 1 - q;  // the link of x whose source is x + c_q
-            const uint8_t kb = kind_at(a.kind, aa_nb<L, q>(Ly, wraps, e, x, y, z, 1));
+            const uint8_t kb = kind_at(a.kind, nb.template elem<q, 1>());
             if (kb >= KIND_COND0 && kb < KIND_INERT)
-                plane_ref<B32>(m, q, Ly.plane, e) =
+                nb.template at<q, q, 0>() =
                     IO::template from_calc<j>(rule_value<L, M, j>(cond_at(a.conds, kb - KIND_COND0), os, own[q]));
         });
     }
 }
 
-template <class L, Mode M, bool B32>
-__global__ void __launch_bounds__(256) k_aa_oe(StepArgs a, int tpp, double rxl) {
+template <class L, Mode M, class Nb>
+__device__ __forceinline__ void aa_oe_cell(const StepArgs& a, const Nb& nb) {
     using IO = Io<M, L>;
-    using T = typename IO::T;
     using Calc = typename IO::Calc;
     constexpr int Q = L::Q;
-    const FieldLayout& Ly = a.L;
-    int x, y, z;
-    if (!aa_tile_cell(Ly, tpp, rxl, x, y, z)) return;
-    using I = typename ElemIdx<B32>::type;
-    const I e = static_cast<I>(cell_elem(Ly, x, y, z));
-    const uint8_t k = kind_at(a.kind, e);
+    const uint8_t k = kind_at(a.kind, nb.e);
     if (k >= KIND_COND0) return;
-    T* __restrict__ m = static_cast<T*>(a.dst);
     Calc f[Q];
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        f[q] = IO::template load<q>(plane_ref<B32>(m, Q - 1 - q, Ly.plane, e));
+        f[q] = IO::template load<q>(nb.template at<Q - 1 - q, q, 0>());
     });
-    aa_collide<L, M>(a, static_cast<int64_t>(e), f);
+    aa_collide<L, M>(a, static_cast<int64_t>(nb.e), f);
     static_for<0, Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
-        plane_ref<B32>(m, q, Ly.plane, e) = IO::template store<q>(f[q]);
+        nb.template at<q, q, 0>() = IO::template store<q>(f[q]);
     });
     if (k == KIND_NEAR) {
-        const bool wraps = aa_wraps(Ly, x, y, z);
         Calc own[Q];
         aa_own<L, M>(f, own);
         const OwnSums<Calc> os = own_sums<L, Calc>(own);
         static_for<0, Q>([&](auto qc) {
             constexpr int q = decltype(qc)::value;
-            const I be = aa_nb<L, q>(Ly, wraps, e, x, y, z, -1);
-            const uint8_t kb = kind_at(a.kind, be);
+            const uint8_t kb = kind_at(a.kind, nb.template elem<q, -1>());
             if (kb >= KIND_COND0 && kb < KIND_INERT)
-                plane_ref<B32>(m, q, Ly.plane, be) =
+                nb.template at<q, q, -1>() =
                     IO::template from_calc<q>(rule_value<L, M, q>(cond_at(a.conds, kb - KIND_COND0), os, own[Q - 1 - q]));
         });
+    }
+}
+
+// Row tiles (tpr > 0, planes under 4 GiB) or the plane tiling of k_cells. The
+// element arithmetic of 2 Q neighbours per lane weighs on 16-bit storage, and
+// a wavefront that spans rows touches lines twice. Plane / row tiles, us per
+// step of a periodic D3Q19 box: fp32 64^3 8.98 / 6.97, 100^3 31.2 / 25.9, 150^3
+// 112 / 93.5, 256^3 495 / 491; fp16 200x150x170 80 / 71.5, 192^3 131 / 109.
+// Plain stores: streaming ones measured 18 % slower at 100^3 and equal
+// elsewhere, write-through ones 1 to 12 % slower.
+template <class L, Mode M, bool B32, bool ROW>
+__global__ void __launch_bounds__(256) k_aa_eo(StepArgs a, int tpp, double rxl, int tpr) {
+    using T = typename Io<M, L>::T;
+    int x, y, z;
+    if constexpr (ROW) {
+        if (row_tile_cell(a.L, tpr, x, y, z)) aa_eo_cell<L, M>(a, AaRow<L, T>(static_cast<T*>(a.dst), a.L, x, y, z));
+    } else {
+        if (aa_tile_cell(a.L, tpp, rxl, x, y, z))
+            aa_eo_cell<L, M>(a, AaPlane<L, T, B32>(static_cast<T*>(a.dst), a.L, x, y, z));
+    }
+}
+
+template <class L, Mode M, bool B32, bool ROW>
+__global__ void __launch_bounds__(256) k_aa_oe(StepArgs a, int tpp, double rxl, int tpr) {
+    using T = typename Io<M, L>::T;
+    int x, y, z;
+    if constexpr (ROW) {
+        if (row_tile_cell(a.L, tpr, x, y, z)) aa_oe_cell<L, M>(a, AaRow<L, T>(static_cast<T*>(a.dst), a.L, x, y, z));
+    } else {
+        if (aa_tile_cell(a.L, tpp, rxl, x, y, z))
+            aa_oe_cell<L, M>(a, AaPlane<L, T, B32>(static_cast<T*>(a.dst), a.L, x, y, z));
     }
 }
 

@@ -43,11 +43,20 @@ struct OpsImpl {
                            a, p.tpp, p.rxl);
     }
 
+    static dim3 row_grid(const StepArgs& a, const StepPlan& p) {
+        return dim3(static_cast<uint32_t>((static_cast<int64_t>(p.tpr) * a.L.yl + 3) / 4), static_cast<uint32_t>(a.L.zl));
+    }
+
     template <int... Vs>
     static hipError_t step_impl(const StepArgs& a, const StepPlan& p, hipStream_t s, EventLog* log) {
         // (the dual-number run steps in rows)
         if constexpr (M != Mode::DUAL64) if (p.cells) {
-            if (p.freeslip) {
+            if (p.tpr && !p.freeslip) {
+                if (a.cached)
+                    hipLaunchKernelGGL((k_cell_rows<L, M, true>), row_grid(a, p), dim3(256), 0, s, a, p.tpr);
+                else
+                    hipLaunchKernelGGL((k_cell_rows<L, M, false>), row_grid(a, p), dim3(256), 0, s, a, p.tpr);
+            } else if (p.freeslip) {
                 if (p.idx32)
                     launch_cells<true, true>(a, p, s);
                 else
@@ -203,10 +212,15 @@ struct OpsImpl {
     template <bool B32>
     static void launch_aa(const StepArgs& a, const StepPlan& p, int phase, hipStream_t s) {
         const dim3 grid(static_cast<uint32_t>(p.nblocks_cells));
-        if (phase == 0)
-            hipLaunchKernelGGL((k_aa_eo<L, M, B32>), grid, dim3(256), 0, s, a, p.tpp, p.rxl);
+        if (B32 && p.tpr && phase < 2) {
+            if (phase == 0)
+                hipLaunchKernelGGL((k_aa_eo<L, M, true, true>), row_grid(a, p), dim3(256), 0, s, a, 0, 0.0, p.tpr);
+            else
+                hipLaunchKernelGGL((k_aa_oe<L, M, true, true>), row_grid(a, p), dim3(256), 0, s, a, 0, 0.0, p.tpr);
+        } else if (phase == 0)
+            hipLaunchKernelGGL((k_aa_eo<L, M, B32, false>), grid, dim3(256), 0, s, a, p.tpp, p.rxl, 0);
         else if (phase == 1)
-            hipLaunchKernelGGL((k_aa_oe<L, M, B32>), grid, dim3(256), 0, s, a, p.tpp, p.rxl);
+            hipLaunchKernelGGL((k_aa_oe<L, M, B32, false>), grid, dim3(256), 0, s, a, p.tpp, p.rxl, 0);
         else
             hipLaunchKernelGGL((k_aa_swap<L, M, B32>), grid, dim3(256), 0, s, a, p.tpp, p.rxl);
     }
