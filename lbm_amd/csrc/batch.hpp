@@ -60,6 +60,7 @@ struct BatchArgs {
     int parity;        // src = buf[parity], dst = buf[parity ^ 1]
     int materialised;  // the step pulls stored boundary values
     int freeslip;      // some domain has a FreeSlip condition (cell tiles built with its rule)
+    int rev;           // walk the cell tiles from the last to the first (StepArgs::rev)
     int cached;        // StepArgs::cached, for the buffers of all domains
     int idx32;         // every domain's plane is under 4 GiB (cell tiles use 32-bit byte offsets)
     int nxcd;          // L2 domains the launch's blocks are dealt to (cell tiles: tile_walk)

@@ -53,6 +53,7 @@ struct BatchAdjArgs {
     int* status;                             // hist_forward: non-finite flags as BatchArgs::status
     int terminal;
     int materialised;
+    int rev;     // hist_*: walk the tiles from the last to the first (StepArgs::rev)
     int cached;  // StepArgs::cached, for what one launch reads and writes of all domains
     int idx32;  // every domain's plane is under 4 GiB (32-bit byte offsets)
     int nxcd;   // L2 domains the launch's blocks are dealt to (tile_walk)

@@ -631,7 +631,8 @@ int lbm_set_tuning(lbm_domain* d, int vec, int block_x) {
 static int run_steps(lbm_domain* d, uint64_t nsteps, EventLog* log) {
     if (d->aa) {
         for (uint64_t t = 0; t < nsteps; ++t) {
-            const StepArgs a = d->args(d->buf[0], d->buf[0], d->materialised ? 1 : 0);
+            StepArgs a = d->args(d->buf[0], d->buf[0], d->materialised ? 1 : 0);
+            a.rev = turns_back(d->field_bytes) ? d->aa_phase : 0;
             hipError_t e = d->ops->aa_step(a, d->plan, d->aa_phase, d->stream);
             if (log) log->mark(d->stream, 0);
             if (e != hipSuccess) return fail(LBM_ERR_HIP, std::string("step launch: ") + hipGetErrorString(e));

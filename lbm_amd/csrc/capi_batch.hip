@@ -180,6 +180,7 @@ hipError_t enqueue(lbm_batch* b, uint64_t nsteps, int parity, int mat) {
         std::max<int64_t>(1, std::min<int64_t>((b->nnear + 127) / 128, static_cast<int64_t>(b->ncu) * 16)));
     for (uint64_t s = 0; s < nsteps; ++s) {
         a.parity = parity;
+        a.rev = turns_back(2 * b->field_bytes) ? parity : 0;
         a.materialised = (s == 0) ? mat : 0;
         const hipError_t e = b->ops->launch(a, b->V, b->kernel, grid_bulk, grid_near, b->stream);
         if (e != hipSuccess) return e;
@@ -783,6 +784,7 @@ int lbm_batch_adj_forward(lbm_batch_tape* t, double* J) {
         for (uint64_t s = 1; s <= t->T; ++s) {
             a.hist_step = static_cast<int64_t>(s);
             a.parity = parity;
+            a.rev = turns_back(2 * b->field_bytes) ? parity : 0;
             a.materialised = s == 1 ? mat : 0;
             HIPCHK(t->ops->hist_forward(a, grid_for(t), b->stream));
             parity ^= 1;
@@ -890,6 +892,7 @@ int lbm_batch_adj_backward(lbm_batch_tape* t, double* grad_wall) {
                 a.hist_step = static_cast<int64_t>(s);
                 a.mu_in_slot = mu_slot(t, static_cast<int>((s + 1) & 1));
                 a.mu_out_slot = mu_slot(t, static_cast<int>(s & 1));
+                a.rev = turns_back(2 * b->field_bytes) ? static_cast<int>(s & 1) : 0;
                 a.terminal = (s == t->T) ? 1 : 0;
                 a.materialised = (s == 1 && t->start_mat) ? 1 : 0;
                 HIPCHK(t->ops->hist_backward(a, grid, b->stream));

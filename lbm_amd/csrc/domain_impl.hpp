@@ -116,6 +116,19 @@ inline size_t elem_size(Mode m) {
 // tiles measured faster streamed as well.
 inline int fits_cache(size_t bytes) { return bytes > (size_t{32} << 20) && bytes <= (size_t{256} << 20) ? 1 : 0; }
 
+// Whether the cell-tile kernels sweep every other step backwards. A step then
+// starts with the cells the last one wrote last, which the memory-side cache
+// still holds, where a forward sweep finds it full of the field's other end.
+// Below the 32 MiB of all L2s the turn only moves tiles to another L2 than the
+// one that wrote them. Forward only / turning, us per step, D3Q19: in place
+// fp32 64^3 (20 MB) 7.1 / 7.1, 150^3 95 / 86, 200x150x170 (388 MB) 195 / 126,
+// 256^3 491 / 454; cavity singly 16^3 9.9 / 10.5 (so not turned), fp64 64^3
+// 19.9 / 19.3, fp32 64^3 14.3 / 13.6; 64 mixed cavities 272 / 252, their
+// adjoint 306 + 316 / 294 + 299. The row kernel and the passes, whose output
+// is streamed past the cache, gain nothing from it (256^3 fp32 458 / 461 and
+// 288 / 287, walled pass at 192^3 155 / 157) and always sweep forwards.
+inline int turns_back(size_t bytes) { return bytes > (size_t{32} << 20) ? 1 : 0; }
+
 inline int64_t roundup(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 // L2 domains (XCDs) of a gfx950 device with ncu compute units: 32 CUs and
@@ -191,6 +204,7 @@ struct lbm_domain {
         a.lmask = d_lmask;
         a.lcond = d_lcond;
         a.cached = fits_cache(2 * field_bytes);
+        a.rev = (src == buf[1] && turns_back(2 * field_bytes)) ? 1 : 0;
         a.span32 = field_bytes < (size_t{1} << 32) ? 1 : 0;
         a.rlist = d_rlist;
         a.nr = nr;

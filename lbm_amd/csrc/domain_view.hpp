@@ -85,6 +85,7 @@ struct StepArgs {
     void* dst;
     const uint8_t* kind;
     const uint32_t* lmask;  // link word per element
+    int rev;                // cell tiles: sweep from the last plane to the first (turns_back)
     int cached;             // the buffers a step reads and writes fit the memory-side cache
     int span32;             // a whole buffer is under 4 GiB: 32-bit byte offsets across planes
     // per element: for a NEAR cell, the condition index shared by every link

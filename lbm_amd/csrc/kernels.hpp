@@ -690,10 +690,10 @@ struct RowNb {
 
 // Row tiles: wavefront w of z plane 1 + blockIdx.y takes cells 64 (w mod tpr)
 // + 1 .. of row 1 + w / tpr. False past the row or the plane.
-__device__ __forceinline__ bool row_tile_cell(const FieldLayout& L, int tpr, int& x, int& y, int& z) {
+__device__ __forceinline__ bool row_tile_cell(const FieldLayout& L, int tpr, int rev, int& x, int& y, int& z) {
     const int w = static_cast<int>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
     y = 1 + w / tpr;
-    z = 1 + static_cast<int>(blockIdx.y);
+    z = rev ? L.zl - static_cast<int>(blockIdx.y) : 1 + static_cast<int>(blockIdx.y);
     x = 1 + (w % tpr) * 64 + static_cast<int>(threadIdx.x & 63);
     return y <= L.yl && x <= L.xl;
 }
@@ -959,14 +959,15 @@ constexpr int cells_min_blocks() {
 template <class L, Mode M, bool CACHED>
 __global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cell_rows(StepArgs a, int tpr) {
     int x, y, z;
-    if (row_tile_cell(a.L, tpr, x, y, z)) any_cell<L, M, false, true, CACHED, false, true>(a, x, y, z);
+    if (row_tile_cell(a.L, tpr, a.rev, x, y, z)) any_cell<L, M, false, true, CACHED, false, true>(a, x, y, z);
 }
 
 template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false>
 __global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cells(StepArgs a, int tpp, double rxl) {
     const int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
-    const int z = 1 + static_cast<int>(w / tpp);
+    int z = 1 + static_cast<int>(w / tpp);
     if (z > a.L.zl) return;
+    if (a.rev) z = a.L.zl + 1 - z;
     const int64_t c = (w % tpp) * 64 + (threadIdx.x & 63);
     const int64_t xl = a.L.xl;
     if (c >= xl * a.L.yl) return;

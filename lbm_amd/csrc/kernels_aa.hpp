@@ -49,10 +49,11 @@ __device__ __forceinline__ bool aa_wraps(const FieldLayout& Ly, int x, int y, in
 }
 
 // Cell (x, y, z) of this lane in the k_cells tiling; false past the domain.
-__device__ __forceinline__ bool aa_tile_cell(const FieldLayout& Ly, int tpp, double rxl, int& x, int& y, int& z) {
+__device__ __forceinline__ bool aa_tile_cell(const FieldLayout& Ly, int tpp, double rxl, int rev, int& x, int& y, int& z) {
     const int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     z = 1 + static_cast<int>(w / tpp);
     if (z > Ly.zl) return false;
+    if (rev) z = Ly.zl + 1 - z;
     const int64_t c = (w % tpp) * 64 + (threadIdx.x & 63);
     const int64_t xl = Ly.xl;
     if (c >= xl * Ly.yl) return false;
@@ -213,9 +214,9 @@ __global__ void __launch_bounds__(256) k_aa_eo(StepArgs a, int tpp, double rxl, 
     using T = typename Io<M, L>::T;
     int x, y, z;
     if constexpr (ROW) {
-        if (row_tile_cell(a.L, tpr, x, y, z)) aa_eo_cell<L, M>(a, AaRow<L, T>(static_cast<T*>(a.dst), a.L, x, y, z));
+        if (row_tile_cell(a.L, tpr, a.rev, x, y, z)) aa_eo_cell<L, M>(a, AaRow<L, T>(static_cast<T*>(a.dst), a.L, x, y, z));
     } else {
-        if (aa_tile_cell(a.L, tpp, rxl, x, y, z))
+        if (aa_tile_cell(a.L, tpp, rxl, a.rev, x, y, z))
             aa_eo_cell<L, M>(a, AaPlane<L, T, B32>(static_cast<T*>(a.dst), a.L, x, y, z));
     }
 }
@@ -225,9 +226,9 @@ __global__ void __launch_bounds__(256) k_aa_oe(StepArgs a, int tpp, double rxl, 
     using T = typename Io<M, L>::T;
     int x, y, z;
     if constexpr (ROW) {
-        if (row_tile_cell(a.L, tpr, x, y, z)) aa_oe_cell<L, M>(a, AaRow<L, T>(static_cast<T*>(a.dst), a.L, x, y, z));
+        if (row_tile_cell(a.L, tpr, a.rev, x, y, z)) aa_oe_cell<L, M>(a, AaRow<L, T>(static_cast<T*>(a.dst), a.L, x, y, z));
     } else {
-        if (aa_tile_cell(a.L, tpp, rxl, x, y, z))
+        if (aa_tile_cell(a.L, tpp, rxl, a.rev, x, y, z))
             aa_oe_cell<L, M>(a, AaPlane<L, T, B32>(static_cast<T*>(a.dst), a.L, x, y, z));
     }
 }
@@ -241,7 +242,7 @@ __global__ void __launch_bounds__(256) k_aa_swap(StepArgs a, int tpp, double rxl
     constexpr int Q = L::Q;
     const FieldLayout& Ly = a.L;
     int x, y, z;
-    if (!aa_tile_cell(Ly, tpp, rxl, x, y, z)) return;
+    if (!aa_tile_cell(Ly, tpp, rxl, a.rev, x, y, z)) return;
     using I = typename ElemIdx<B32>::type;
     const I e = static_cast<I>(cell_elem(Ly, x, y, z));
     if (kind_at(a.kind, e) >= KIND_COND0) return;

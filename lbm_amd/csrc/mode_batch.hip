@@ -67,7 +67,7 @@ __global__ void __launch_bounds__(256) k_batch_cells(BatchArgs b) {
     const int lane = threadIdx.x & 63;
     const TileWalk w = tile_walk(b.ntiles, b.nxcd);
     for (int t = w.t; t < w.end; t += w.stride) {
-        const TileRef tr = b.tiles[t];
+        const TileRef tr = b.tiles[b.rev ? b.ntiles - 1 - t : t];
         const BatchView& v = b.views[tr.dom];
         const int z = 1 + tr.local / v.tpp;
         const int c = (tr.local % v.tpp) * 64 + lane;

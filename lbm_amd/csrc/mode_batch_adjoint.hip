@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(256) k_badj_hist_forward(BatchAdjArgs b) {
     const int lane = threadIdx.x & 63;
     const TileWalk w = tile_walk(b.ntiles, b.nxcd);
     for (int t = w.t; t < w.end; t += w.stride) {
-        const TileRef tr = b.tiles[t];
+        const TileRef tr = b.tiles[b.rev ? b.ntiles - 1 - t : t];
         const BatchAdjView& v = b.views[tr.dom];
         int x, y, z;
         if (!tile_cell(v, tr.local, lane, x, y, z)) continue;
@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(256) k_badj_hist_backward(BatchAdjArgs b) {
     const int lane = threadIdx.x & 63;
     const TileWalk w = tile_walk(b.ntiles, b.nxcd);
     for (int t = w.t; t < w.end; t += w.stride) {
-        const TileRef tr = b.tiles[t];
+        const TileRef tr = b.tiles[b.rev ? b.ntiles - 1 - t : t];
         const BatchAdjView& v = b.views[tr.dom];
         int x, y, z;
         if (!tile_cell(v, tr.local, lane, x, y, z)) continue;
