@@ -56,7 +56,7 @@ int lbm_moments(lbm_domain* d, double* rho, double* u) {
         d->desc.device, d->stream, n, 4 * sizeof(double),
         [&](void* slot, int64_t i0, int64_t m, hipStream_t s) {
             double* v = static_cast<double*>(slot);
-            return d->ops->moments(d->L, d->buf[d->cur], v, v + m, i0, m, s);
+            return d->ops->moments(d->L, d->buf[d->cur], rho ? v : nullptr, u ? v + m : nullptr, i0, m, s);
         },
         [&](const char* v, int64_t i0, int64_t m) {
             const size_t part = static_cast<size_t>(m) * sizeof(double);

@@ -73,11 +73,17 @@ __device__ __forceinline__ void load_cell_f64(const FieldLayout& Ly, const void*
 // density() then velocity(density) of interior cells, x fastest
 // (include/io/vtk.hpp:62-73). EXACT64 follows the reference sums; the shifted
 // modes return rho = 1 + sum g and u = sum c g / rho evaluated in double.
-// Cells i0 .. i0 + n - 1; rho and u hold those cells.
+// Cells i0 .. i0 + n - 1; rho and u hold those cells and may lie in host
+// memory: the block's velocities, 3 values a cell, are put in order in LDS, so
+// that every store instruction fills whole lines.
 template <class L, Mode M>
-__global__ void k_moments(FieldLayout Ly, const void* src, double* rho, double* u, int64_t i0, int64_t n) {
-    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i >= n) return;
+__global__ void __launch_bounds__(256) k_moments(FieldLayout Ly, const void* src, double* rho, double* u, int64_t i0,
+                                                 int64_t n) {
+    __shared__ double su[3 * 256];
+    const int tid = static_cast<int>(threadIdx.x);
+    const int64_t b0 = blockIdx.x * int64_t{256};
+    const int m = n - b0 < 256 ? static_cast<int>(n - b0) : 256;  // cells of this block
+    const int64_t i = b0 + (tid < m ? tid : m - 1);               // (idle threads repeat the last one)
     const int64_t c = i0 + i;
     const int x = 1 + static_cast<int>(c % Ly.xl);
     const int y = 1 + static_cast<int>((c / Ly.xl) % Ly.yl);
@@ -101,12 +107,12 @@ __global__ void k_moments(FieldLayout Ly, const void* src, double* rho, double* 
         v[1] = jy / r;
         v[2] = jz / r;
     }
-    if (rho) rho[i] = r;
-    if (u) {
-        u[3 * i + 0] = v[0];
-        u[3 * i + 1] = v[1];
-        u[3 * i + 2] = v[2];
-    }
+    if (rho && tid < m) rho[i] = r;
+    if (!u) return;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) su[3 * tid + k] = v[k];
+    __syncthreads();
+    for (int j = tid; j < 3 * m; j += 256) u[3 * b0 + j] = su[j];
 }
 
 // Block sum of 4 doubles over a 256-thread block; result valid in thread 0.
@@ -172,15 +178,22 @@ static __global__ void __launch_bounds__(256) k_sum_partials(const double* parti
 }
 
 // Interior fluid cells i0 .. i0 + n - 1 <- feq(rho, u); rho and u hold those
-// cells, x fastest.
+// cells, x fastest (in host memory or on the device, as k_moments).
 template <class L, Mode M>
-__global__ void k_init_eq(FieldLayout Ly, void* dst_, const uint8_t* kind, const double* rho,
-                          const double* u, int64_t i0, int64_t n) {
+__global__ void __launch_bounds__(256) k_init_eq(FieldLayout Ly, void* dst_, const uint8_t* kind, const double* rho,
+                                                 const double* u, int64_t i0, int64_t n) {
     using IO = Io<M, L>;
     using T = typename IO::T;
     using Calc = typename IO::Calc;
-    const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-    if (i >= n) return;
+    __shared__ double su[3 * 256];
+    const int tid = static_cast<int>(threadIdx.x);
+    const int64_t b0 = blockIdx.x * int64_t{256};
+    const int m = n - b0 < 256 ? static_cast<int>(n - b0) : 256;
+    for (int j = tid; j < 3 * m; j += 256) su[j] = u[3 * b0 + j];
+    const int64_t i = b0 + (tid < m ? tid : m - 1);
+    const double r = rho[i];
+    __syncthreads();
+    if (tid >= m) return;
     const int64_t c = i0 + i;
     const int x = 1 + static_cast<int>(c % Ly.xl);
     const int y = 1 + static_cast<int>((c / Ly.xl) % Ly.yl);
@@ -188,8 +201,7 @@ __global__ void k_init_eq(FieldLayout Ly, void* dst_, const uint8_t* kind, const
     const int64_t e = cell_elem(Ly, x, y, z);
     if (kind[e] >= KIND_COND0) return;
     T* dst = static_cast<T*>(dst_);
-    const double r = rho[i];
-    const double v[3] = {u[3 * i + 0], u[3 * i + 1], u[3 * i + 2]};
+    const double v[3] = {su[3 * tid + 0], su[3 * tid + 1], su[3 * tid + 2]};
     static_for<0, L::Q>([&](auto qc) {
         constexpr int q = decltype(qc)::value;
         double val;
