@@ -629,7 +629,7 @@ int batch_adj_create(lbm_batch* b, uint64_t nsteps, uint64_t k1, uint64_t k2, bo
     if (automatic) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
-            nsteps <= std::min(total_b / 4, free_b / 2) / record &&
+            nsteps <= std::min(total_b / 4, free_b / 2) / record && nsteps * record + 3 * field_total <= free_b &&
             hipMalloc(&t->hist, nsteps * record) != hipSuccess) {
             (void)hipGetLastError();
             t->hist = nullptr;
@@ -776,7 +776,7 @@ int lbm_batch_adj_forward(lbm_batch_tape* t, double* J) {
         a.tiles = t->d_tiles;
         a.ntiles = t->ntiles;
         a.idx32 = b->all_idx32 ? 1 : 0;
-    a.cached = fits_cache(2 * b->field_bytes);
+        a.cached = fits_cache(2 * b->field_bytes);
         a.nxcd = 1;  // (as the forward step)
         a.status = b->d_status;
         HIPCHK(hipMemcpyAsync(t->d_views, t->views.data(), sizeof(BatchAdjView) * t->views.size(),
