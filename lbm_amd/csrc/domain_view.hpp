@@ -107,7 +107,11 @@ struct StepArgs {
     double g[3];
     // Kernels built with HIST: 4 Calc values (drho, u) of the incoming
     // populations per interior cell, x fastest, written here by the step (and
-    // by a two-step pass's second step at hist2).
+    // by a two-step pass's second step at hist2). Written and read past the
+    // caches: each value is used once, a whole sweep later, and displaced lines
+    // that the step itself reads again (objective and gradient, plain / non-
+    // temporal: 128^3 porosity, 100 steps 11.8 / 11.5 ms; 64 mixed cavities, 50
+    // steps 30.4 / 29.6 ms).
     void* hist;
     void* hist2;
     // any_cell built with HIST: index of a NEAR cell in the domain's list per

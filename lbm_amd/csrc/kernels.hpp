@@ -927,7 +927,7 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
             f, static_cast<Calc>(a.omega), Calc(0), Calc(0), Calc(0), Calc(0), HIST ? mom.v : nullptr));
         if constexpr (HIST) {
             const Mom4Raw<Calc> m = {mom.v[0], mom.v[1], mom.v[2], mom.v[3]};
-            glob(static_cast<Mom4Raw<Calc>*>(a.hist))[cell_index(Ly, x, y, z)] = m;
+            __builtin_nontemporal_store(m, &glob(static_cast<Mom4Raw<Calc>*>(a.hist))[cell_index(Ly, x, y, z)]);
         }
     }
     static_for<0, Q>([&](auto qc) {

@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(256) k_adj2(AdjArgs a, int ntx, int nty, int z
                 constexpr int q = decltype(qc)::value;
                 lam[q] = tb_at(mi + q * plane, zs3[1 + L::cz(q)] + ys[1 + L::cy(q)] + xs[1 + L::cx(q)]);
             });
-            const Mom4<float> m = hist[cell_index(Ly, gx[k], gy[k], gz)];
+            const Mom4<float> m = hist[cell_index(Ly, gx[k], gy[k], gz)];  // (ring cells again by other blocks)
             float al = 0.0f;
             if constexpr (BRINK) al = tb_at(alpha, zs3[1] + ys[1] + xs[1]);
             const float d = adjoint_relax<L, float, BRINK>(m.v[0], m.v[1], m.v[2], m.v[3], lam, mu, omega, al, tgx, tgy,
@@ -192,7 +192,9 @@ __global__ void __launch_bounds__(256) k_adj2(AdjArgs a, int ntx, int nty, int z
                         lam[q] = lds[S::template slot<q>()][c];
                     });
                     const uint32_t eb = 4u * (static_cast<uint32_t>(Ly.off) + ox) + pz * zo + py * oy;
-                    const Mom4<float> m = hist2[cell_index(Ly, ox, oy, zo)];
+                    const Mom4Raw<float> mr =
+                        __builtin_nontemporal_load(reinterpret_cast<const Mom4Raw<float>*>(hist2) + cell_index(Ly, ox, oy, zo));
+                    const Mom4<float> m = {{mr[0], mr[1], mr[2], mr[3]}};
                     float al = 0.0f;
                     if constexpr (BRINK) al = tb_at(alpha, eb);
                     const float d = adjoint_relax<L, float, BRINK>(m.v[0], m.v[1], m.v[2], m.v[3], lam, mu, omega, al,

@@ -577,7 +577,7 @@ __device__ __forceinline__ void adj_hist_cell(const AdjArgs& a, const uint32_t* 
         return elem_at<B32>(Ly, wrap_if(x + sgn * L::cx(q), Ly.xl, Ly.per[0]),
                             wrap_if(y + sgn * L::cy(q), Ly.yl, Ly.per[1]), wrap_if(z + sgn * L::cz(q), Ly.zl, Ly.per[2]));
     };
-    const Mom4Raw<Calc> m = glob(static_cast<const Mom4Raw<Calc>*>(a.hist))[cell_index(Ly, x, y, z)];
+    const Mom4Raw<Calc> m = __builtin_nontemporal_load(&glob(static_cast<const Mom4Raw<Calc>*>(a.hist))[cell_index(Ly, x, y, z)]);
     uint32_t lm = 0, walls = 0;  // links; links to moving walls
     int lc = LCOND_MIXED;
     if (near) {

@@ -206,7 +206,7 @@ __global__ void __launch_bounds__(256) k_bulk2(StepArgs a, int ntx, int nty, int
                 // tile cells of the chunk, each by its own block
                 if (zs >= z0 && zs <= z1 && pi[k] >= 0 && pi[k] < TB_TX && pj[k] >= 0 && pj[k] < TB_TY &&
                     x0 + pi[k] <= Ly.xl && y0 + pj[k] <= Ly.yl)
-                    static_cast<Mom4<Calc>*>(a.hist)[cell_index(Ly, x0 + pi[k], y0 + pj[k], zs)] = mom;
+                    put<Put::Stream>(static_cast<Mom4<Calc>*>(a.hist) + cell_index(Ly, x0 + pi[k], y0 + pj[k], zs), mom);
             }
             static_for<0, Q>([&](auto qc) {
                 constexpr int q = decltype(qc)::value;
@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(256) k_bulk2(StepArgs a, int ntx, int nty, int
                     if constexpr (BRINK) al = alpha[eb / TS];
                     Mom4<Calc> mom;
                     tb_collide<L, M, BRINK>(a, f, al, HIST ? mom.v : nullptr);
-                    if constexpr (HIST) static_cast<Mom4<Calc>*>(a.hist2)[cell_index(Ly, ox, oy, zo)] = mom;
+                    if constexpr (HIST) put<Put::Stream>(static_cast<Mom4<Calc>*>(a.hist2) + cell_index(Ly, ox, oy, zo), mom);
                     static_for<0, Q>([&](auto qc) {
                         constexpr int q = decltype(qc)::value;
                         put<CACHED ? Put::Through : Put::Stream>(tb_ptr(dst + q * plane, eb), IO::template store<q>(f[q]));
