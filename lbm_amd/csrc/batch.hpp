@@ -21,6 +21,7 @@ struct BatchView {
     const uint8_t* kind;
     const uint32_t* lmask;
     const uint8_t* lcond;
+    const uint32_t* rword;
     int span32;           // StepArgs::span32
     const Cond* conds;
     double tau, omega;

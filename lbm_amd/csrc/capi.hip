@@ -229,6 +229,7 @@ void free_device(lbm_domain* d) {
     d->d_kind = nullptr;
     d->d_lmask = nullptr;
     d->d_lcond = nullptr;
+    d->d_rword = nullptr;
     d->d_blist = nullptr;
     d->d_rlist = nullptr;
     d->d_conds = nullptr;
@@ -519,10 +520,11 @@ int lbm_finalize(lbm_domain* d) {
 
     // Cell kinds in the padded device layout, the NEAR list, the link masks
     // of NEAR cells (bit q: the source x - c_q is not fluid) and the
-    // condition their links share (LCOND_MIXED where they differ).
+    // condition their links share (LCOND_MIXED where they differ); rule words.
     std::vector<uint8_t> kind(static_cast<size_t>(L.plane), KIND_INERT);
     std::vector<uint32_t> lmask(static_cast<size_t>(L.plane), LINK_NOT_FLUID);
     std::vector<uint8_t> lcond(static_cast<size_t>(L.plane), LCOND_MIXED);
+    std::vector<uint32_t> rword(static_cast<size_t>(L.plane), 0u);
     std::vector<CellCoord> blist, rlist;
     uint64_t nfluid = 0, nbulk = 0, nonbulk_interior = 0;
     for (int z = 0; z < d->nz; ++z)
@@ -540,6 +542,8 @@ int lbm_finalize(lbm_domain* d) {
                 ++nfluid;
                 uint32_t m = 0;
                 int shared = -1;  // condition of the links so far (-2: more than one)
+                int rshared = -1;  // of those that are not NoSlip
+                uint32_t rm = 0;
                 for (int q = 0; q < Q; ++q) {
                     const int64_t sx = d->wrapc(x - lat.c[q][0], 0);
                     const int64_t sy = d->wrapc(y - lat.c[q][1], 1);
@@ -548,11 +552,18 @@ int lbm_finalize(lbm_domain* d) {
                     if (hs != 0) {
                         m |= 1u << q;
                         const int ci = cond_map[hs - 1];
-                        if (uniq[ci].kind != LBM_BC_NOSLIP) m |= LINK_RULES;
+                        if (uniq[ci].kind != LBM_BC_NOSLIP) {
+                            m |= LINK_RULES;
+                            rm |= 1u << q;
+                            rshared = rshared == -1 ? ci : (rshared == ci ? ci : -2);
+                        }
                         shared = shared == -1 ? ci : (shared == ci ? ci : -2);
                     }
                 }
                 lmask[e] = m;
+                if (rm)
+                    rword[e] = rm | (rshared >= 0 ? std::min(static_cast<uint32_t>(rshared), RULE_SLOW) : RULE_SLOW)
+                                        << RULE_SHIFT;
                 if (m) {
                     kind[e] = KIND_NEAR;
                     if (shared >= 0) lcond[e] = static_cast<uint8_t>(shared);
@@ -567,14 +578,19 @@ int lbm_finalize(lbm_domain* d) {
 
     HIPCHK(hipMemcpyAsync(d->d_kind, kind.data(), kind.size(), hipMemcpyHostToDevice, d->stream));
     if (!d->d_lmask) {
-        const size_t bytes = lmask.size() * (sizeof(uint32_t) + sizeof(uint8_t));
+        const size_t words = lmask.size() * (rlist.empty() ? 1 : 2);
+        const size_t bytes = words * sizeof(uint32_t) + lcond.size();
         HIPCHK(hipMalloc(&d->d_lmask, bytes));
-        d->d_lcond = reinterpret_cast<uint8_t*>(d->d_lmask + lmask.size());
+        if (!rlist.empty()) d->d_rword = d->d_lmask + lmask.size();
+        d->d_lcond = reinterpret_cast<uint8_t*>(d->d_lmask + words);
         d->device_bytes += bytes;
     }
     HIPCHK(hipMemcpyAsync(d->d_lmask, lmask.data(), lmask.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
                           d->stream));
     HIPCHK(hipMemcpyAsync(d->d_lcond, lcond.data(), lcond.size(), hipMemcpyHostToDevice, d->stream));
+    if (d->d_rword)
+        HIPCHK(hipMemcpyAsync(d->d_rword, rword.data(), rword.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
+                              d->stream));
     d->nb = static_cast<int64_t>(blist.size());
     if (d->nb) {
         d->nr = static_cast<int64_t>(rlist.size());

@@ -88,6 +88,7 @@ int configure(lbm_batch* b, int V, int bx_policy, int bpc, int kernel) {
         v.kind = d->d_kind;
         v.lmask = d->d_lmask;
         v.lcond = d->d_lcond;
+        v.rword = d->d_rword;
         v.span32 = d->field_bytes < (size_t{1} << 32) ? 1 : 0;
         v.conds = d->d_conds;
         v.tau = d->desc.tau;
@@ -678,6 +679,7 @@ int batch_adj_create(lbm_batch* b, uint64_t nsteps, uint64_t k1, uint64_t k2, bo
         v.kind = d->d_kind;
         v.lmask = d->d_lmask;
         v.lcond = d->d_lcond;
+        v.rword = d->d_rword;
         v.span32 = d->field_bytes < (size_t{1} << 32) ? 1 : 0;
         v.conds = d->d_conds;
         v.tau = d->desc.tau;

@@ -159,6 +159,7 @@ struct lbm_domain {
     uint8_t* d_kind = nullptr;
     uint32_t* d_lmask = nullptr;  // per element: link word (domain_view.hpp)
     uint8_t* d_lcond = nullptr;   // per element: their shared condition (same allocation, after d_lmask)
+    uint32_t* d_rword = nullptr;  // rule words where nr > 0, else null (same allocation)
     CellCoord* d_blist = nullptr;
     int64_t nb = 0;
     CellCoord* d_rlist = nullptr;  // NEAR cells with LINK_RULES (after d_blist, same allocation)
@@ -203,6 +204,7 @@ struct lbm_domain {
         a.kind = d_kind;
         a.lmask = d_lmask;
         a.lcond = d_lcond;
+        a.rword = d_rword;
         a.cached = fits_cache(2 * field_bytes);
         a.rev = (src == buf[1] && turns_back(2 * field_bytes)) ? 1 : 0;
         a.span32 = field_bytes < (size_t{1} << 32) ? 1 : 0;

@@ -36,6 +36,12 @@ constexpr uint32_t LINK_BITS = (1u << 27) - 1;
 constexpr uint32_t LINK_RULES = 1u << 30;
 constexpr uint32_t LINK_NOT_FLUID = 1u << 31;
 
+// Rule word of a cell with LINK_RULES (StepArgs::rword): bits q < Q the links
+// whose condition is not NoSlip, and above them the index of that condition
+// where it is the same for all of them and below RULE_SLOW, else RULE_SLOW.
+constexpr int RULE_SHIFT = 27;
+constexpr uint32_t RULE_SLOW = 31;
+
 // Boundary-condition kinds, numbered as in include/lbm_hip.h.
 enum : int {
     BC_NOSLIP = 1,
@@ -92,6 +98,7 @@ struct StepArgs {
     // of its mask, or LCOND_MIXED where they differ (edges and corners);
     // may be null (every cell then takes the per-link path)
     const uint8_t* lcond;
+    const uint32_t* rword;  // rule word per element; null in a domain without LINK_RULES cells
     const CellCoord* blist;  // cells of kind NEAR
     int64_t nb;
     const CellCoord* rlist;  // those with LINK_RULES

@@ -65,7 +65,13 @@ __global__ void __launch_bounds__(256) k_emit_rules(StepArgs a) {
     T* __restrict__ buf = static_cast<T*>(a.dst);
     const uint32_t e = elem_at<true>(Ly, c.x, c.y, c.z);
     const uint32_t lm = glob(a.lmask)[e];
-    const int lc = glob(a.lcond)[e];
+    // (as in near_rules)
+    uint32_t rm = a.rword ? glob(a.rword)[e] : RULE_SLOW << RULE_SHIFT;
+    int lc = static_cast<int>(rm >> RULE_SHIFT);
+    if (lc == static_cast<int>(RULE_SLOW) || !(lm & LINK_RULES)) {
+        lc = glob(a.lcond)[e];
+        rm = lm;
+    }
     Calc own[Q];
     OwnAcc<L, Calc> acc;
     static_for<0, Q>([&](auto qc) {
@@ -76,7 +82,7 @@ __global__ void __launch_bounds__(256) k_emit_rules(StepArgs a) {
     T rv[Q];
     auto put = [&](auto qc, Calc v) {
         constexpr int q = decltype(qc)::value;
-        rv[q] = IO::template from_calc<q>(v);
+        rv[q] = IO::template from_calc<q>(pick_bits(((rm >> q) & 1u) != 0, v, own[Q - 1 - q]));
     };
     auto finv = [&](auto qc) { return own[Q - 1 - decltype(qc)::value]; };
     if (lc != LCOND_MIXED) {

@@ -14,6 +14,7 @@ __device__ __forceinline__ StepArgs view_args(const BatchView& v, int parity, in
     a.kind = v.kind;
     a.lmask = v.lmask;
     a.lcond = v.lcond;
+    a.rword = v.rword;
     a.span32 = v.span32;
     a.cached = cached;
     a.conds = v.conds;

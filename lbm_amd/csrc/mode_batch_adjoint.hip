@@ -57,7 +57,8 @@ __global__ void __launch_bounds__(256) k_badj_recompute(BatchAdjArgs b) {
         a.kind = v.kind;
         a.lmask = v.lmask;
         a.lcond = v.lcond;
-    a.span32 = v.span32;
+        a.rword = v.rword;
+        a.span32 = v.span32;
         a.cached = b.cached;
         a.conds = v.conds;
         a.materialised = b.materialised;
@@ -131,7 +132,8 @@ __global__ void __launch_bounds__(256) k_badj_hist_forward(BatchAdjArgs b) {
         a.kind = v.kind;
         a.lmask = v.lmask;
         a.lcond = v.lcond;
-    a.span32 = v.span32;
+        a.rword = v.rword;
+        a.span32 = v.span32;
         a.cached = b.cached;
         a.conds = v.conds;
         a.materialised = b.materialised;
