@@ -178,7 +178,7 @@ __global__ void __launch_bounds__(256) k_badj_hist_backward(BatchAdjArgs b) {
         const Calc* r = record<Calc>(v, b.hist_step);
         a.hist = r;
         a.cached = b.cached;
-        adj_hist_cell<L, M, B32>(a, v.lmask, v.lcond, x, y, z, e, k == KIND_NEAR, r + record_near(v), v.near_idx, v.gw);
+        adj_hist_cell<L, M, B32>(a, v.lmask, v.rword, x, y, z, e, k == KIND_NEAR, r + record_near(v), v.near_idx, v.gw);
     }
 }
 
