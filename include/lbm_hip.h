@@ -147,7 +147,10 @@ int lbm_get_pdf(lbm_domain* d, double* out);
  * the next step pulls the written values from non-fluid cells as stored. */
 int lbm_set_pdf(lbm_domain* d, const double* in);
 /* Extension: every interior fluid cell <- feq(rho, u) from x-fastest
- * interior arrays rho[xl*yl*zl], u[3*xl*yl*zl] (host pointers). */
+ * interior arrays rho[xl*yl*zl], u[3*xl*yl*zl] (host pointers). In a domain
+ * with boundary cells every non-fluid cell goes back to the values it is
+ * created with, so the run that follows is that of a new domain, whatever the
+ * domain did before and in whichever layout. */
 int lbm_init_equilibrium(lbm_domain* d, const double* rho, const double* u);
 
 /* Replaces Cell::density() / Cell::velocity(density) of every interior cell

@@ -78,12 +78,16 @@ __global__ void __launch_bounds__(256) k_copy_planes(const float2* __restrict__ 
     }
 }
 
-template <class T>
-__global__ void k_fill_planes(T* buf, int64_t plane, int q, const double* values) {
-    const int64_t n = plane * q;
-    for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
+// One value per direction plane (grid y), passed by value: no allocation, no wait.
+struct PlaneValues {
+    double v[27];
+};
+__global__ void k_fill_planes(double* buf, int64_t plane, PlaneValues values) {
+    const double v = values.v[blockIdx.y];
+    double* p = buf + blockIdx.y * plane;
+    for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < plane;
          i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-        buf[i] = static_cast<T>(values[i / plane]);
+        p[i] = v;
 }
 
 }  // namespace
@@ -248,13 +252,12 @@ int fill_initial(lbm_domain* d, void* buf) {
         HIPCHK(hipMemsetAsync(buf, 0, d->field_bytes, d->stream));
         return LBM_OK;
     }
-    DeviceTemp dv;
-    HIPCHK(hipMalloc(&dv.p, sizeof(double) * d->Q));
-    HIPCHK(hipMemcpyAsync(dv.p, d->lat.w, sizeof(double) * d->Q, hipMemcpyHostToDevice, d->stream));
-    hipLaunchKernelGGL(k_fill_planes<double>, dim3(4096), dim3(256), 0, d->stream,
-                       static_cast<double*>(buf), d->L.plane, d->Q, static_cast<const double*>(dv.p));
+    PlaneValues values{};
+    for (int q = 0; q < d->Q; ++q) values.v[q] = d->lat.w[q];
+    const uint32_t gx = static_cast<uint32_t>(std::min<int64_t>((d->L.plane + 255) / 256, 1024));
+    hipLaunchKernelGGL(k_fill_planes, dim3(gx, static_cast<uint32_t>(d->Q)), dim3(256), 0, d->stream,
+                       static_cast<double*>(buf), d->L.plane, values);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(d->stream));
     return LBM_OK;
 }
 

@@ -24,9 +24,12 @@ int lbm_init_equilibrium(lbm_domain* d, const double* rho, const double* u) {
     if (!d->finalized) return fail(LBM_ERR_STATE, "call lbm_finalize first (fluid cells are needed)");
     if (!rho || !u) return fail(LBM_ERR_ARG, "null input");
     const int64_t n = static_cast<int64_t>(d->L.xl) * d->L.yl * d->L.zl;
-    if (d->aa) {
-        // boundary cells back to the weights, as the two-buffer layout holds them
-        if (int rc = fill_initial(d, d->buf[0])) return rc;
+    // A restart: the next step pulls stored values from non-fluid cells, so
+    // these go back to what a new domain holds. By now they may hold rule
+    // values of an earlier state (in the in-place layout always; else where a
+    // two-step pass or a reader of whole cells wrote them) or of lbm_set_pdf.
+    if (d->nb || d->aa) {
+        if (int rc = fill_initial(d, d->buf[d->cur])) return rc;
         d->aa_phase = 0;
     }
     const hipError_t e = staged_write(

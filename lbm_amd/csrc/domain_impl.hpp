@@ -59,17 +59,6 @@ private:
     std::vector<hipEvent_t> ev_;
 };
 
-// Device memory owned by a scope: freed when it ends, error returns included.
-struct DeviceTemp {
-    void* p = nullptr;
-    DeviceTemp() = default;
-    ~DeviceTemp() {
-        if (p) (void)hipFree(p);
-    }
-    DeviceTemp(const DeviceTemp&) = delete;
-    DeviceTemp& operator=(const DeviceTemp&) = delete;
-};
-
 struct HostCond {
     int kind;
     double vel[3];
