@@ -150,7 +150,7 @@ def walled_case(capi, name: str, q: int, mode: str, dims, tau: float, sc, steps:
         sc.apply(d)
         d.finalize()
         if spp == 2:
-            out["default_steps_per_pass"] = d.info()["steps_per_pass"]
+            out["default_steps_per_launch"] = d.info()["steps_per_launch"]
         d.set_time_blocking(spp)
         info = d.info()
         d.step(warmup)
@@ -180,7 +180,7 @@ def walled_case(capi, name: str, q: int, mode: str, dims, tau: float, sc, steps:
         if spp == 1:
             out.update({"lattice": f"D3Q{q}", "storage": mode, "shape": list(dims), "tau": tau, "steps": steps,
                         "interior_cells": interior, "fluid_cells": fluid, "near_cells": info["ncells_near"]})
-    head = out["pass"] if out["default_steps_per_pass"] == 2 else out["single_step"]
+    head = out["pass"] if out["default_steps_per_launch"] == 2 else out["single_step"]
     out["mlups"] = head["mlups"]
     return out
 

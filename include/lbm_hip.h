@@ -357,11 +357,17 @@ typedef struct lbm_info {
     int nconds;                /* distinct boundary conditions */
     int cell_tiles;            /* 1: steps run as 64-cell tiles per wavefront (k_cells) */
     int layout;                /* enum lbm_layout */
-    int steps_per_pass;        /* 2: lbm_step runs pairs of steps as one pass (the automatic setting
-                                * steps domains below the sizes of lbm_set_time_blocking singly) */
+    int steps_per_pass;        /* 2: a two-step pass applies to the domain under the current setting
+                                * (lbm_get_steps_per_launch: whether lbm_step takes it) */
     int z_chunk;               /* planes per block of the two-step pass */
 } lbm_info;
 int lbm_get_info(lbm_domain* d, lbm_info* info);
+/* Steps that one launch of lbm_step advances a finalized domain by: 2 where it
+ * runs pairs of steps as one pass, 1 where it steps singly, as the automatic
+ * setting does with the domains named at lbm_set_time_blocking although a pass
+ * applies. (An odd last step is single in either form, and so is a walled
+ * domain's first step after initialisation or lbm_set_pdf.) */
+int lbm_get_steps_per_launch(lbm_domain* d, int* steps);
 
 /* Tuning. vec = 0 (default): domains with boundary cells step as 64-cell
  * tiles per wavefront, every cell kind in one kernel; bulk-only domains use

@@ -98,6 +98,7 @@ SIGNATURES = [
     ("lbm_batch_adj_backward", c_int, [c_void_p, POINTER(c_double)]),
     ("lbm_batch_adj_timing", c_int, [c_void_p, POINTER(c_double)]),
     ("lbm_get_info", c_int, [c_void_p, POINTER(Info)]),
+    ("lbm_get_steps_per_launch", c_int, [c_void_p, POINTER(c_int)]),
     ("lbm_set_tuning", c_int, [c_void_p, c_int, c_int]),
     ("lbm_set_time_blocking", c_int, [c_void_p, c_int, c_int]),
     ("lbm_set_index_width", c_int, [c_void_p, c_int]),
@@ -304,9 +305,14 @@ class Domain:
         return out
 
     def info(self) -> dict:
+        """lbm_info's fields; of a finalized domain also steps_per_launch."""
         i = Info()
         _check(load().lbm_get_info(self._h, byref(i)))
-        return {k: getattr(i, k) for k, _ in Info._fields_}
+        out = {k: getattr(i, k) for k, _ in Info._fields_}
+        n = c_int()
+        if load().lbm_get_steps_per_launch(self._h, byref(n)) == 0:
+            out["steps_per_launch"] = n.value
+        return out
 
     def set_tuning(self, vec: int = 0, block_x: int = 0) -> None:
         _check(load().lbm_set_tuning(self._h, vec, block_x))

@@ -647,6 +647,10 @@ int lbm_set_tuning(lbm_domain* d, int vec, int block_x) {
     return LBM_OK;
 }
 
+static int steps_per_launch(const lbm_domain* d) {
+    return (d->plan.pairs || d->plan.wpairs) && !d->plan.small_single ? 2 : 1;
+}
+
 static int run_steps(lbm_domain* d, uint64_t nsteps, EventLog* log) {
     if (d->aa) {
         for (uint64_t t = 0; t < nsteps; ++t) {
@@ -661,7 +665,7 @@ static int run_steps(lbm_domain* d, uint64_t nsteps, EventLog* log) {
         return LBM_OK;
     }
     uint64_t t = 0;
-    const bool passes = !d->plan.small_single;
+    const bool passes = steps_per_launch(d) == 2;
     if (d->plan.wpairs && passes) {
         // the first step after set-up pulls stored boundary values: single
         if (d->materialised && t < nsteps) {
@@ -921,6 +925,13 @@ int lbm_get_info(lbm_domain* d, lbm_info* info) {
     info->layout = d->aa ? LBM_LAYOUT_AA : LBM_LAYOUT_AB;
     info->steps_per_pass = (d->plan.pairs || d->plan.wpairs) ? 2 : 1;
     info->z_chunk = d->plan.tb_zc;
+    return LBM_OK;
+}
+
+int lbm_get_steps_per_launch(lbm_domain* d, int* steps) {
+    if (!d || !steps) return fail(LBM_ERR_ARG, "null argument");
+    if (!d->finalized) return fail(LBM_ERR_STATE, "call lbm_finalize first");
+    *steps = steps_per_launch(d);
     return LBM_OK;
 }
 
