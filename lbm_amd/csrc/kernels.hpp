@@ -38,6 +38,24 @@ struct alignas(sizeof(T) * V) VecT {
     T v[V];
 };
 
+// Pulled values, converted by here. bf16's conversion is one shift, which the
+// compiler otherwise moves to the uses behind the branches that follow, and
+// then holds raw and converted values at once: k_cell_rows D3Q19 spilled 32 of
+// its 80 registers, D3Q27 took 136 (3 waves per SIMD), k_bulk D3Q27 172 (2).
+// With this and through_storage's they take 80 (no spills), 110 and 133. us a
+// step, without / with: D3Q19 64^3 sphere channel 19.3 / 13.8, 160x150x140
+// 122 / 92, walls across z 28x60x50 11.4 / 9.4, D3Q27 periodic 192x160x128
+// singly 126 / 101 (but D3Q27 channels of 32^3 12.4 / 13.5).
+// (An empty asm at each load made the loads wait for one another: the walled
+// two-step pass took 1.4 times as long.)
+template <Mode M, int Q, class Calc>
+__device__ __forceinline__ void converted(Calc (&f)[Q]) {
+    if constexpr (M == Mode::BF16) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) __asm__("" : "+v"(f[q]));
+    }
+}
+
 // drho and u of one cell and step (StepArgs::hist).
 template <class Calc>
 struct alignas(16) Mom4 {
@@ -276,6 +294,8 @@ __device__ __forceinline__ bool bulk_cells(const StepArgs& a, int x0, int y, int
     // the loads above are issued before this test (every row they touch lies
     // inside the ghosted box), so the kind lookup costs no extra round trip
     if (!any) return true;
+#pragma unroll
+    for (int i = 0; i < V; ++i) converted<M>(f[i]);
 
     Calc alpha[V];
     if constexpr (BRINK) {
@@ -922,6 +942,7 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
     } else {
         pull_all<L, M, B32>(src, Ly.plane, e, links, a.span32, wrap_src, f);
     }
+    converted<M>(f);
     if (rules) {
         near_rules<L, M, FS, B32>(a, e, x, y, z, f);
         if constexpr (HIST) {  // (read by the moving walls' gradient only)

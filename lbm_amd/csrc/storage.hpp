@@ -142,6 +142,10 @@ struct Io {
     // rounds, in every kernel alike.
     template <int q>
     __device__ __forceinline__ static Calc through_storage(Calc g) {
+        // (bf16: without the empty asm the compiler folds the round trip of a
+        // value that was loaded, and then keeps raw and converted values at
+        // once in the cell kernels: see converted())
+        if constexpr (M == Mode::BF16) __asm__("" : "+v"(g));
         return load<q>(from_calc<q>(g));
     }
 };
