@@ -984,13 +984,19 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
 }
 
 // Blocks of 256 per CU the cell-tile kernel is compiled for: 6 (80 VGPRs)
-// with 32- and 16-bit storage up to D3Q19; no bound with 64-bit arithmetic,
-// whose values take twice the registers, or with D3Q27, where 80 VGPRs
-// spill.
-template <class L, Mode M>
+// with 32- and 16-bit storage up to D3Q19, 4 in fp64 reference order; no bound
+// with F64S, whose values take twice the registers, or with D3Q27, where 80
+// VGPRs spill. FreeSlip's rule takes more: D3Q19 spilled 39 (fp32), 20 (fp16),
+// 12 (bf16) and 76 (fp64) registers under those bounds, which cost more than
+// the waves gave: there 5 blocks, and no bound in fp64. us a step, those
+// bounds / these, half-slip cavities: 28x30x30 fp32 16.4 / 14.5, fp16 16.4 /
+// 14.7, bf16 16.1 / 14.6, fp64 18.7 / 15.8; 160x128x128 103 / 92, 73.8 / 70.5,
+// 75.2 / 71.1, 194 / 179.
+template <class L, Mode M, bool FS>
 constexpr int cells_min_blocks() {
-    if (M == Mode::EXACT64) return L::Q > 19 ? 1 : 4;
-    return (M == Mode::F64S || M == Mode::DUAL64 || L::Q > 19) ? 1 : 6;
+    if (M == Mode::EXACT64) return L::Q > 19 || (FS && L::Q > 15) ? 1 : 4;
+    if (M == Mode::F64S || L::Q > 19) return 1;
+    return FS && L::Q > 15 ? 5 : 6;
 }
 
 // Cell-tile kernels. k_cell_rows (planes under 4 GiB, no FreeSlip): row tiles,
@@ -1003,13 +1009,13 @@ constexpr int cells_min_blocks() {
 // (x fastest) of the z plane 1 + w / tpp, for packed rows and the rest.
 // CACHED: the output policy, built in (a branch on it spilled registers).
 template <class L, Mode M, bool CACHED>
-__global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cell_rows(StepArgs a, int tpr) {
+__global__ void __launch_bounds__(256, (cells_min_blocks<L, M, false>())) k_cell_rows(StepArgs a, int tpr) {
     int x, y, z;
     if (row_tile_cell(a.L, tpr, a.rev, x, y, z)) any_cell<L, M, false, true, CACHED, false, true>(a, x, y, z);
 }
 
 template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false>
-__global__ void __launch_bounds__(256, (cells_min_blocks<L, M>())) k_cells(StepArgs a, int tpp, double rxl) {
+__global__ void __launch_bounds__(256, (cells_min_blocks<L, M, FS>())) k_cells(StepArgs a, int tpp, double rxl) {
     const int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     int z = 1 + static_cast<int>(w / tpp);
     if (z > a.L.zl) return;

@@ -63,8 +63,11 @@ __global__ void __launch_bounds__(256) k_batch_bulk(BatchArgs b) {
 // range of the list); each lane takes one cell of its tile.
 // The tile index is wavefront-uniform; readfirstlane states it, so the tile
 // and the domain view are read into scalar registers once per wavefront.
+// FreeSlip's rule takes 130 registers, two more than leave 4 wavefronts per
+// SIMD room: 40 half-slip cavities fp32 86.1 -> 79.8 us a step with the bound,
+// fp16 80.6 -> 71.7 (F64S needs 199).
 template <class L, Mode M, bool FS, bool B32, bool CACHED = false>
-__global__ void __launch_bounds__(256) k_batch_cells(BatchArgs b) {
+__global__ void __launch_bounds__(256, (FS && M != Mode::F64S ? 4 : 1)) k_batch_cells(BatchArgs b) {
     const int lane = threadIdx.x & 63;
     const TileWalk w = tile_walk(b.ntiles, b.nxcd);
     for (int t = w.t; t < w.end; t += w.stride) {
