@@ -48,11 +48,11 @@ __global__ void __launch_bounds__(256) k_batch_bulk(BatchArgs b) {
             bool nl[V];
 #pragma unroll
             for (int i = 0; i < V; ++i) nl[i] = false;
-            finite = bulk_cells<L, M, V, true, false>(a, x0, y, z, nl);
+            finite = bulk_cells<L, M, V, true, false, false, false>(a, x0, y, z, nl);
             for (int i = 0; i < V; ++i)
                 if (nl[i]) finite &= near_cell<L, M>(a, x0 + i, y, z);
         } else {
-            finite = bulk_cells<L, M, V, true, false>(a, x0, y, z);
+            finite = bulk_cells<L, M, V, true, false, false, false>(a, x0, y, z);
         }
         // every lane that saw a non-finite value writes the same flag
         if (!finite) b.status[tr.dom] = 1;
