@@ -63,6 +63,7 @@ struct BatchArgs {
     int freeslip;      // some domain has a FreeSlip condition (cell tiles built with its rule)
     int rev;           // walk the cell tiles from the last to the first (StepArgs::rev)
     int cached;        // StepArgs::cached, for the buffers of all domains
+    int ahead;         // cell tiles: any_cell's AHEAD form where built (fp32)
     int idx32;         // every domain's plane is under 4 GiB (cell tiles use 32-bit byte offsets)
     int nxcd;          // L2 domains the launch's blocks are dealt to (cell tiles: tile_walk)
     // one flag per domain, set to 1 by a step in which a fluid cell of the

@@ -132,6 +132,18 @@ int make_plan(lbm_domain* d) {
     // wavefront long, from where on their tiles are at least half full; a
     // launch's y extent, at most 65535, counts the planes.
     p.tpr = (p.idx32 && !d->compact && d->L.zl <= 65535 && d->L.xl >= 32) ? (d->L.xl + 63) / 64 : 0;
+    const int64_t cells = plane_cells * d->L.zl;
+    // Few x lines with a near-boundary cell: most wavefronts have no links.
+    const bool open_lines = 3 * d->near_lines <= static_cast<int64_t>(d->L.yl) * d->L.zl;
+    // There, in a domain whose launch lasts as long as one wavefront's chain of
+    // accesses, pulls that wait for the link word only add to the chain. us per
+    // step, link word first / AHEAD: periodic box 12^3 fp32 7.77 / 6.85, bf16
+    // 7.30 / 6.85, F64S 8.09 / 7.37, 28 x 60 x 50 fp32 9.85 / 8.78, fp64 13.2 /
+    // 11.7 (but 64^3 fp16 10.1 / 10.7); walls across z only, 28 x 60 x 50 fp32
+    // 10.5 / 9.4, bf16 9.35 / 9.05. D3Q27 in 32 and 16 bits loses with walls:
+    // 12^3 fp32 8.61 / 8.80, bf16 8.98 / 9.23. With links in every line (cavity,
+    // walls across x) AHEAD takes up to 25 % longer.
+    p.ahead = open_lines && cells < 100000 && (d->nb == 0 || d->Q <= 19 || d->esize == 8);
     p.cells = d->tune_vec == 0 && (d->nb > 0 || d->compact) &&
               p.nblocks_cells <= 0x7fffffffLL && (plane_cells + 63) / 64 <= 0x7fffffffLL;
     if (!p.cells && d->compact && V > 1)
@@ -211,8 +223,7 @@ int make_plan(lbm_domain* d) {
     //   channel around spheres (fluid 0.8): D3Q19 192x96x96 60.5 / 72.7,
     //     256x128x128 171 / 148; D3Q27 91.7 / 120, 258 / 243;
     //   pipe 208x100x100: D3Q19 63.1 / 86.0, D3Q27 90.9 / 153.
-    const uint64_t cells = static_cast<uint64_t>(d->L.xl) * d->L.yl * d->L.zl;
-    const uint64_t least = !walled ? 3 * 65536 : (d->n_fluid == cells ? 600000 : 3000000);
+    const int64_t least = !walled ? 3 * 65536 : (d->n_fluid == static_cast<uint64_t>(cells) ? 600000 : 3000000);
     // With walls the cell tiles also gain more from output kept in the
     // memory-side cache (Put::Keep) than the pass does.
     p.small_single = d->tune_pass == 0 && (cells < least || (walled && fits_cache(2 * d->field_bytes)));
@@ -595,6 +606,8 @@ int lbm_finalize(lbm_domain* d) {
         HIPCHK(hipMemcpyAsync(d->d_rword, rword.data(), rword.size() * sizeof(uint32_t), hipMemcpyHostToDevice,
                               d->stream));
     d->nb = static_cast<int64_t>(blist.size());
+    for (size_t i = 0; i < blist.size(); ++i)
+        d->near_lines += i == 0 || blist[i].y != blist[i - 1].y || blist[i].z != blist[i - 1].z;
     if (d->nb) {
         d->nr = static_cast<int64_t>(rlist.size());
         blist.insert(blist.end(), rlist.begin(), rlist.end());

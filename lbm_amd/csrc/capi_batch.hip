@@ -33,6 +33,7 @@ struct lbm_batch {
     bool any_compact = false;   // some domain packs its rows: row kernels take V = 1 only
     bool any_freeslip = false;  // some domain has a FreeSlip condition
     size_t field_bytes = 0;     // one buffer of every domain
+    uint64_t packed_cells = 0;  // cells in packed rows that end at walls
     bool all_idx32 = true;      // every domain's plane is under 4 GiB
     int64_t near_cells = 0;     // NEAR cells of all domains
     BatchView* d_views = nullptr;
@@ -168,6 +169,7 @@ hipError_t enqueue(lbm_batch* b, uint64_t nsteps, int parity, int mat) {
     a.freeslip = b->any_freeslip ? 1 : 0;
     a.idx32 = b->all_idx32 ? 1 : 0;
     a.cached = fits_cache(2 * b->field_bytes);
+    a.ahead = b->bpc ? 0 : pulls_ahead(b->doms[0]->mode, 2 * b->field_bytes, b->packed_cells, b->ncells);
     // the forward step keeps the plain walk: grouping tiles by L2 domain
     // measured slower there (512 cavities of 16-96 cells a side: 2.43
     // against 2.10 ms per step), while it pays in the adjoint's kernels
@@ -231,6 +233,7 @@ int lbm_batch_create(lbm_domain* const* domains, int n, lbm_batch** out) {
     for (const lbm_domain* d : b->doms) {
         b->ncells += static_cast<uint64_t>(d->L.xl) * d->L.yl * d->L.zl;
         b->field_bytes += d->field_bytes;
+        if (d->compact && !d->L.per[0]) b->packed_cells += static_cast<uint64_t>(d->L.xl) * d->L.yl * d->L.zl;
         b->any_compact |= d->compact;
         b->any_freeslip |= d->plan.freeslip;
         b->all_idx32 &= d->plan.idx32;

@@ -118,6 +118,20 @@ inline int fits_cache(size_t bytes) { return bytes > (size_t{32} << 20) && bytes
 // 288 / 287, walled pass at 192^3 155 / 157) and always sweep forwards.
 inline int turns_back(size_t bytes) { return bytes > (size_t{32} << 20) ? 1 : 0; }
 
+// Whether the batched cell tiles step in any_cell's AHEAD form: fp32 sets far
+// beyond the caches in which most cells (packed_cells of them) lie in packed
+// rows between walls. us a step, link word first / AHEAD, one block per four
+// tiles. Uneven cavities of 16 to 96 cells a side, MiB of all buffers: 64 (992)
+// 243 / 252, 128 (1841) 468 / 470, 150 (2027) 525 / 516, 192 (2699) 711 / 694,
+// 256 (3634) 997 / 945, 512 (7737) 2160 / 1980. Other sets of 2 to 6.5 GiB:
+// edges 12 to 40 1085 / 1032, 40 to 62 1186 / 1057; in padded rows, edges 64 to
+// 160 1474 / 1600, 40 cavities of 70^3 619 / 629, 40 periodic boxes of 70^3 633
+// / 729. A persistent grid loses (512: 2779 / 2933), and so do the other
+// storages (512: fp16 1381 / 1397, F64S 3437 / 3571).
+inline int pulls_ahead(Mode m, size_t bytes, uint64_t packed_cells, uint64_t cells) {
+    return m == Mode::F32 && bytes > (size_t{2} << 30) && 2 * packed_cells > cells ? 1 : 0;
+}
+
 inline int64_t roundup(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 
 // L2 domains (XCDs) of a gfx950 device with ncu compute units: 32 CUs and
@@ -153,6 +167,7 @@ struct lbm_domain {
     int64_t nb = 0;
     CellCoord* d_rlist = nullptr;  // NEAR cells with LINK_RULES (after d_blist, same allocation)
     int64_t nr = 0;
+    int64_t near_lines = 0;  // x lines with a NEAR cell
     Cond* d_conds = nullptr;
     int nconds_dev = 0;
     void* d_alpha = nullptr;

@@ -789,21 +789,13 @@ __device__ __forceinline__ void pull_all(const typename Io<M, L>::T* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// One interior cell of any kind, for kernels that hand every cell of a region
-// to a thread (the cell tiles). Non-fluid cells return at once. The link word
-// says which directions bounce back (pull_all); a cell with a link of another
-// rule pulls every direction plainly (sources wrapped along periodic axes;
-// along a walled axis the source may be a ghost or solid cell) and then
-// replaces the values pulled from non-fluid sources by their boundary values
-// (as near_cell). All lanes collide and store together. The bits
-// equal those of bulk_cells / near_cell for the same cell. B32 takes the
-// cell's own and plain-pull addresses as 32-bit byte offsets (planes under
-// 4 GiB). Returns false when a fluid cell read a NaN or infinite value.
 // The pulls of a NEAR cell x with LINK_RULES (element e, ghosted-box coordinates x, y, z)
 // from non-fluid sources, f[q] for every link q of its mask, replaced by
 // their boundary values, from x's stored values in a.src (the reference's
 // boundary pass folded into the pull).
-template <class L, Mode M, bool FS, bool B32>
+// ALL: any NEAR cell, those with NoSlip links only among them; the condition
+// that all links share comes first.
+template <class L, Mode M, bool FS, bool B32, bool ALL = false>
 __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B32>::type e, int x, int y, int z,
                                            typename Io<M, L>::Calc (&f)[L::Q]) {
     using IO = Io<M, L>;
@@ -819,59 +811,63 @@ __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B
         return IO::template to_calc<kk>(plane_ref<B32>(src, kk, Ly.plane, e));
     };
     const uint32_t lm = glob(a.lmask)[e] & LINK_BITS;
-    if constexpr (M != Mode::DUAL64) {
-        // Every link that is not NoSlip under one condition (not FreeSlip,
-        // whose rule reads other cells), as on edges between a lid and walls:
-        // one branch on its kind, then that family's loads go out together,
-        // where the path below waits for two lookups a link, one link after
-        // the other. The values are rule_value's (same functions). (A caller
-        // without the rule words takes the path below.) With the shared path
-        // only where all links agree, and not in fp64: 16^3 fp32 cavity, 10
-        // steps with moments 140 -> 90 us, 64^3 fp64 cavity, 100 steps 2.21 ->
-        // 1.83 ms, 250 x 54 x 54 fp16 pipe 2.51 -> 2.14 ms, 30 mixed cavities
-        // 89.9 -> 83.6 us a step, D3Q27 sphere channel 192 x 96 x 96, 100
-        // steps 10.8 -> 10.4 ms.
-        uint32_t rm = 0;
-        int rc = LCOND_MIXED;
-        if (a.rword) {
-            const uint32_t rw = glob(a.rword)[e];
+    // Every link that is not NoSlip under one condition (not FreeSlip,
+    // whose rule reads other cells), as on edges between a lid and walls:
+    // one branch on its kind, then that family's loads go out together,
+    // where the path below waits for two lookups a link, one link after
+    // the other. The values are rule_value's (same functions). (A caller
+    // without the rule words takes the path below.) With the shared path
+    // only where all links agree, and not in fp64: 16^3 fp32 cavity, 10
+    // steps with moments 140 -> 90 us, 64^3 fp64 cavity, 100 steps 2.21 ->
+    // 1.83 ms, 250 x 54 x 54 fp16 pipe 2.51 -> 2.14 ms, 30 mixed cavities
+    // 89.9 -> 83.6 us a step, D3Q27 sphere channel 192 x 96 x 96, 100
+    // steps 10.8 -> 10.4 ms.
+    uint32_t rm = lm;
+    int rc = LCOND_MIXED;
+    if constexpr (ALL) rc = glob(a.lcond)[e];
+    if (rc == LCOND_MIXED && a.rword) {
+        const uint32_t rw = glob(a.rword)[e];
+        if ((rw >> RULE_SHIFT) != RULE_SLOW) {
             rm = rw;
             rc = static_cast<int>(rw >> RULE_SHIFT);
-            if (rc == static_cast<int>(RULE_SLOW)) {  // (more than RULE_SLOW conditions)
-                rc = glob(a.lcond)[e];
-                rm = lm;
-            }
+        } else if constexpr (!ALL) {  // (more than RULE_SLOW conditions)
+            rc = glob(a.lcond)[e];
         }
-        if (rc != LCOND_MIXED) {
-            const GCond& cd = cond_at(a.conds, rc);
-            const int ck = cd.kind;
-            // (the reference-order outflow rule, two equilibria a link, is
-            // built once, below)
-            if ((!FS || ck != BC_FREESLIP) && (M != Mode::EXACT64 || ck == BC_MOVINGWALL || ck == BC_INFLOW)) {
-                auto finv = [&](auto qc) { return own(std::integral_constant<int, Q - 1 - decltype(qc)::value>{}); };
-                auto put = [&](auto qc, Calc own_inv, Calc v) {
-                    constexpr int q = decltype(qc)::value;
-                    const Calc b = pick_bits(((rm >> q) & 1u) != 0, v, own_inv);  // (NoSlip: the own value)
-                    f[q] = pick_bits(((lm >> q) & 1u) != 0, IO::template through_storage<q>(b), f[q]);
-                };
-                if (ck == BC_MOVINGWALL) {
-                    static_for<0, Q>([&](auto qc) {
-                        const Calc w = finv(qc);
-                        put(qc, w, rule_value<L, M, decltype(qc)::value, RULE_MOVINGWALL>(cd, os, w));
-                    });
-                } else if (ck == BC_INFLOW) {
-                    static_for<0, Q>([&](auto qc) {
-                        const Calc w = finv(qc);
-                        put(qc, w, rule_value<L, M, decltype(qc)::value, RULE_INFLOW>(cd, os, w));
-                    });
-                } else if constexpr (M != Mode::EXACT64) {  // Outflow, Pressure (NoSlip-only cells do not come here)
-                    static_for<0, Q>([&](auto qc) {
-                        const Calc w = finv(qc);
-                        put(qc, w, outflow_rule<L, Calc, decltype(qc)::value>(os, w, cd));
-                    });
-                }
-                return;
+    }
+    if (rc != LCOND_MIXED) {
+        const GCond& cd = cond_at(a.conds, rc);
+        const int ck = cd.kind;
+        // (the reference-order outflow rule, two equilibria a link, is
+        // built once, below)
+        if ((!FS || ck != BC_FREESLIP) && (M != Mode::EXACT64 || (ALL && ck == BC_NOSLIP) || ck == BC_MOVINGWALL || ck == BC_INFLOW)) {
+            auto finv = [&](auto qc) { return own(std::integral_constant<int, Q - 1 - decltype(qc)::value>{}); };
+            auto put = [&](auto qc, Calc own_inv, Calc v) {
+                constexpr int q = decltype(qc)::value;
+                const Calc b = pick_bits(((rm >> q) & 1u) != 0, v, own_inv);  // (NoSlip: the own value)
+                f[q] = pick_bits(((lm >> q) & 1u) != 0, IO::template through_storage<q>(b), f[q]);
+            };
+            if (ck == BC_MOVINGWALL) {
+                static_for<0, Q>([&](auto qc) {
+                    const Calc w = finv(qc);
+                    put(qc, w, rule_value<L, M, decltype(qc)::value, RULE_MOVINGWALL>(cd, os, w));
+                });
+            } else if (ck == BC_INFLOW) {
+                static_for<0, Q>([&](auto qc) {
+                    const Calc w = finv(qc);
+                    put(qc, w, rule_value<L, M, decltype(qc)::value, RULE_INFLOW>(cd, os, w));
+                });
+            } else if (ALL && ck == BC_NOSLIP) {
+                static_for<0, Q>([&](auto qc) {
+                    const Calc w = finv(qc);
+                    put(qc, w, w);
+                });
+            } else if constexpr (M != Mode::EXACT64) {  // Outflow, Pressure
+                static_for<0, Q>([&](auto qc) {
+                    const Calc w = finv(qc);
+                    put(qc, w, outflow_rule<L, Calc, decltype(qc)::value>(os, w, cd));
+                });
             }
+            return;
         }
     }
     static_for<0, Q>([&](auto qc) {
@@ -890,9 +886,24 @@ __device__ __forceinline__ void near_rules(const StepArgs& a, typename ElemIdx<B
     });
 }
 
+// One interior cell of any kind, for kernels that hand every cell of a region
+// to a thread (the cell tiles). Non-fluid cells return at once. The link word
+// says which directions bounce back (pull_all); a cell with a link of another
+// rule pulls every direction plainly (sources wrapped along periodic axes;
+// along a walled axis the source may be a ghost or solid cell) and then
+// replaces the values pulled from non-fluid sources by their boundary values
+// (as near_cell). All lanes collide and store together. The bits
+// equal those of bulk_cells / near_cell for the same cell. B32 takes the
+// cell's own and plain-pull addresses as 32-bit byte offsets (planes under
+// 4 GiB). Returns false when a fluid cell read a NaN or infinite value.
 // HIST records drho and u of the incoming populations, and 1 + the sum of
 // the own values of a cell with moving-wall links (StepArgs::hist, rho_own).
-template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false, bool HIST = false, bool ROW = false>
+// AHEAD sends the pulls ahead of the cell's kind, and every NEAR cell takes
+// the values of all its links from near_rules: a shorter chain of accesses for
+// lanes without links, a longer one and Q more loads for those with. make_plan
+// and pulls_ahead (domain_impl.hpp) say where it is taken.
+template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false, bool HIST = false, bool ROW = false,
+          bool AHEAD = false>
 __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z) {
     using IO = Io<M, L>;
     using T = typename IO::T;
@@ -901,15 +912,16 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
     constexpr int Q = L::Q;
     const FieldLayout& Ly = a.L;
     const I e = elem_at<B32>(Ly, x, y, z);
-    const uint32_t w = glob(a.lmask)[e];
+    const uint32_t w = AHEAD ? kind_at(a.kind, e) : glob(a.lmask)[e];  // cell kind (AHEAD) or link word
     const T* __restrict__ src = static_cast<const T*>(a.src);
     T* __restrict__ dst = static_cast<T*>(a.dst);
-    if (w & LINK_NOT_FLUID) return true;
+    if (!AHEAD && (w & LINK_NOT_FLUID)) return true;
 
     // A cell with a link of another rule than NoSlip pulls plainly and
     // patches all its links below; one in its first step pulls stored values.
-    // (Pulls sent ahead of the link word, with the bounced values loaded
-    // afterwards, took 2 to 14 % longer from 64^3 up and no less below.)
+    // (Pulls sent ahead of the link word with only the bounced values loaded
+    // afterwards took 2 to 14 % longer on cavities from 64^3 up, and 2.43
+    // against 1.98 ms in the AHEAD form on 512 batched ones.)
     constexpr I US = B32 ? static_cast<I>(sizeof(T)) : I(1);  // unit of the sources
     Calc f[Q];
     // Away from the faces of periodic axes every source is a fixed element
@@ -927,9 +939,23 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
         return elem_at<B32>(Ly, wrap_if(x - L::cx(q), Ly.xl, Ly.per[0]), wrap_if(y - L::cy(q), Ly.yl, Ly.per[1]),
                             wrap_if(z - L::cz(q), Ly.zl, Ly.per[2])) * US;
     };
-    const bool rules = (w & LINK_RULES) && !a.materialised;
-    const uint32_t links = (rules || a.materialised) ? 0u : w;
-    if constexpr (ROW) {
+    const bool rules = (AHEAD ? w == KIND_NEAR : (w & LINK_RULES) != 0) && !a.materialised;
+    const uint32_t links = (AHEAD || rules || a.materialised) ? 0u : w;
+    if constexpr (AHEAD) {
+        static_assert(!HIST, "plain steps");
+        if constexpr (ROW) {
+            const RowNb<T> nb(Ly, x, y, z);
+            static_for<0, Q>([&](auto qc) {
+                constexpr int q = decltype(qc)::value;
+                f[q] = IO::template load<q>(nb.template at<L, q, -1>(src, Ly.plane));
+            });
+        } else if (!wraps) {
+            pull_plain<L, M, B32>(src, Ly.plane, near_src, f);
+        } else {
+            pull_plain<L, M, B32>(src, Ly.plane, wrap_src, f);
+        }
+        if (w >= KIND_COND0) return true;
+    } else if constexpr (ROW) {
         static_assert(B32, "row tiles take 32-bit offsets");
         const RowNb<T> nb(Ly, x, y, z);
         pull_all<L, M, true>(src, Ly.plane, e, links, a.span32,
@@ -946,7 +972,7 @@ __device__ __forceinline__ bool any_cell(const StepArgs& a, int x, int y, int z)
     }
     converted<M>(f);
     if (rules) {
-        near_rules<L, M, FS, B32>(a, e, x, y, z, f);
+        near_rules<L, M, FS, B32, AHEAD>(a, e, x, y, z, f);
         if constexpr (HIST) {  // (read by the moving walls' gradient only)
             const int lc = glob(a.lcond)[e];
             if (lc == LCOND_MIXED || cond_at(a.conds, lc).kind == BC_MOVINGWALL) {
@@ -1009,14 +1035,15 @@ constexpr int cells_min_blocks() {
 // 131 74.4 / 62.6, 250 136 / 113 (30, half a tile: 20.8 / 22.0).
 // k_cells: wavefront w of the grid takes the 64 cells 64 (w mod tpp) .. + 63
 // (x fastest) of the z plane 1 + w / tpp, for packed rows and the rest.
+// AHEAD: as any_cell (StepPlan::ahead).
 // CACHED: the output policy, built in (a branch on it spilled registers).
-template <class L, Mode M, bool CACHED>
+template <class L, Mode M, bool CACHED, bool AHEAD = false>
 __global__ void __launch_bounds__(256, (cells_min_blocks<L, M, false>())) k_cell_rows(StepArgs a, int tpr) {
     int x, y, z;
-    if (row_tile_cell(a.L, tpr, a.rev, x, y, z)) any_cell<L, M, false, true, CACHED, false, true>(a, x, y, z);
+    if (row_tile_cell(a.L, tpr, a.rev, x, y, z)) any_cell<L, M, false, true, CACHED, false, true, AHEAD>(a, x, y, z);
 }
 
-template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false>
+template <class L, Mode M, bool FS = true, bool B32 = false, bool CACHED = false, bool AHEAD = false>
 __global__ void __launch_bounds__(256, (cells_min_blocks<L, M, FS>())) k_cells(StepArgs a, int tpp, double rxl) {
     const int64_t w = static_cast<int64_t>(blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6);
     int z = 1 + static_cast<int>(w / tpp);
@@ -1035,7 +1062,7 @@ __global__ void __launch_bounds__(256, (cells_min_blocks<L, M, FS>())) k_cells(S
         ++y;
         x -= xl;
     }
-    any_cell<L, M, FS, B32, CACHED>(a, 1 + static_cast<int>(x), 1 + static_cast<int>(y), z);
+    any_cell<L, M, FS, B32, CACHED, false, false, AHEAD>(a, 1 + static_cast<int>(x), 1 + static_cast<int>(y), z);
 }
 
 // Near-boundary kernel: one thread per listed NEAR cell.

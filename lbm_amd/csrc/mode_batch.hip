@@ -66,7 +66,7 @@ __global__ void __launch_bounds__(256) k_batch_bulk(BatchArgs b) {
 // FreeSlip's rule takes 130 registers, two more than leave 4 wavefronts per
 // SIMD room: 40 half-slip cavities fp32 86.1 -> 79.8 us a step with the bound,
 // fp16 80.6 -> 71.7 (F64S needs 199).
-template <class L, Mode M, bool FS, bool B32, bool CACHED = false>
+template <class L, Mode M, bool FS, bool B32, bool CACHED = false, bool AHEAD = false>
 __global__ void __launch_bounds__(256, (FS && M != Mode::F64S ? 4 : 1)) k_batch_cells(BatchArgs b) {
     const int lane = threadIdx.x & 63;
     const TileWalk w = tile_walk(b.ntiles, b.nxcd);
@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(256, (FS && M != Mode::F64S ? 4 : 1)) k_batch_
                 x -= v.L.xl;
             }
             const StepArgs a = view_args(v, b.parity, b.materialised, b.cached);
-            if (!any_cell<L, M, FS, B32, CACHED>(a, 1 + x, 1 + y, z)) b.status[tr.dom] = 1;
+            if (!any_cell<L, M, FS, B32, CACHED, false, false, AHEAD>(a, 1 + x, 1 + y, z)) b.status[tr.dom] = 1;
         }
     }
 }
@@ -123,12 +123,15 @@ struct BatchImpl {
                     else
                         hipLaunchKernelGGL((k_batch_cells<L, M, true, false>), dim3(grid_bulk), dim3(256), 0, s, a);
                 } else {
-                    if (a.idx32 && a.cached)
-                        hipLaunchKernelGGL((k_batch_cells<L, M, false, true, true>), dim3(grid_bulk), dim3(256), 0, s, a);
-                    else if (a.idx32)
-                        hipLaunchKernelGGL((k_batch_cells<L, M, false, true>), dim3(grid_bulk), dim3(256), 0, s, a);
-                    else
+                    if (!a.idx32)
                         hipLaunchKernelGGL((k_batch_cells<L, M, false, false>), dim3(grid_bulk), dim3(256), 0, s, a);
+                    else if (a.cached)
+                        hipLaunchKernelGGL((k_batch_cells<L, M, false, true, true>), dim3(grid_bulk), dim3(256), 0, s, a);
+                    else if (a.ahead)
+                        hipLaunchKernelGGL((k_batch_cells<L, M, false, true, false, M == Mode::F32>), dim3(grid_bulk),
+                                           dim3(256), 0, s, a);
+                    else
+                        hipLaunchKernelGGL((k_batch_cells<L, M, false, true>), dim3(grid_bulk), dim3(256), 0, s, a);
                 }
             }
             return hipGetLastError();

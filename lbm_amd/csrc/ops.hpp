@@ -50,6 +50,7 @@ struct StepPlan {
     bool freeslip;         // a FreeSlip condition exists (cell tiles built with its rule)
     int tpp;               // 64-cell tiles per z plane
     int tpr;               // row tiles: 64-cell tiles per row (0: the plane tiling)
+    bool ahead;            // cell tiles in any_cell's AHEAD form
     int64_t nblocks_cells; // blocks of 4 wavefronts
     double rxl;            // 1 / xl
     // Two steps per pass (k_bulk2): 64 x 8 cell tiles in x-y, tb_zc planes

@@ -37,10 +37,18 @@ struct OpsImpl {
         return true;
     }
 
-    template <bool FS, bool B32, bool CACHED = false>
+    template <bool FS, bool B32, bool CACHED = false, bool AHEAD = false>
     static void launch_cells(const StepArgs& a, const StepPlan& p, hipStream_t s) {
-        hipLaunchKernelGGL((k_cells<L, M, FS, B32, CACHED>), dim3(static_cast<uint32_t>(p.nblocks_cells)), dim3(256), 0, s,
-                           a, p.tpp, p.rxl);
+        hipLaunchKernelGGL((k_cells<L, M, FS, B32, CACHED, AHEAD>), dim3(static_cast<uint32_t>(p.nblocks_cells)), dim3(256),
+                           0, s, a, p.tpp, p.rxl);
+    }
+    // cell tiles without FreeSlip, planes under 4 GiB
+    template <bool CACHED, bool AHEAD>
+    static void launch_cells32(const StepArgs& a, const StepPlan& p, hipStream_t s) {
+        if (p.tpr)
+            hipLaunchKernelGGL((k_cell_rows<L, M, CACHED, AHEAD>), row_grid(a, p), dim3(256), 0, s, a, p.tpr);
+        else
+            launch_cells<false, true, CACHED, AHEAD>(a, p, s);
     }
 
     static dim3 row_grid(const StepArgs& a, const StepPlan& p) {
@@ -51,21 +59,17 @@ struct OpsImpl {
     static hipError_t step_impl(const StepArgs& a, const StepPlan& p, hipStream_t s, EventLog* log) {
         // (the dual-number run steps in rows)
         if constexpr (M != Mode::DUAL64) if (p.cells) {
-            if (p.tpr && !p.freeslip) {
-                if (a.cached)
-                    hipLaunchKernelGGL((k_cell_rows<L, M, true>), row_grid(a, p), dim3(256), 0, s, a, p.tpr);
-                else
-                    hipLaunchKernelGGL((k_cell_rows<L, M, false>), row_grid(a, p), dim3(256), 0, s, a, p.tpr);
-            } else if (p.freeslip) {
+            if (p.freeslip) {
                 if (p.idx32)
                     launch_cells<true, true>(a, p, s);
                 else
                     launch_cells<true, false>(a, p, s);
+            } else if (!p.idx32) {
+                launch_cells<false, false>(a, p, s);
+            } else if (p.ahead) {
+                a.cached ? launch_cells32<true, true>(a, p, s) : launch_cells32<false, true>(a, p, s);
             } else {
-                if (p.idx32)
-                    a.cached ? launch_cells<false, true, true>(a, p, s) : launch_cells<false, true>(a, p, s);
-                else
-                    launch_cells<false, false>(a, p, s);
+                a.cached ? launch_cells32<true, false>(a, p, s) : launch_cells32<false, false>(a, p, s);
             }
             if (log) log->mark(s, 0);
             return hipGetLastError();
