@@ -144,6 +144,15 @@ int make_plan(lbm_domain* d) {
     // 12^3 fp32 8.61 / 8.80, bf16 8.98 / 9.23. With links in every line (cavity,
     // walls across x) AHEAD takes up to 25 % longer.
     p.ahead = open_lines && cells < 100000 && (d->nb == 0 || d->Q <= 19 || d->esize == 8);
+    // In-place layout: row tiles, except with 16-bit storage where the last
+    // tile of a row leaves more than a quarter of the lanes idle and the rows
+    // end at walls: their links then cost more wavefronts than the shared lines
+    // save. Row over plane tiles, time per step, D3Q19 / D3Q27: x = 131 fp16
+    // cavity 1.12 / 1.11, sphere channel 1.13 / 1.07, box 0.92 / 0.89; fp32 1.03
+    // / 1.02, 1.04 / 1.02, 0.89 / 0.88; x = 200 fp16 cavity 1.03 / 0.98, sphere
+    // channel 0.94 / 0.90; x = 250 fp16 cavity 0.94 / 0.90.
+    p.aa_rows = p.tpr > 0 && (d->esize != 2 || d->L.per[0] ||
+                              4 * static_cast<int64_t>(d->L.xl) >= 3 * 64 * static_cast<int64_t>(p.tpr));
     p.cells = d->tune_vec == 0 && (d->nb > 0 || d->compact) &&
               p.nblocks_cells <= 0x7fffffffLL && (plane_cells + 63) / 64 <= 0x7fffffffLL;
     if (!p.cells && d->compact && V > 1)

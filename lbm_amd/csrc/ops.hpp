@@ -51,6 +51,7 @@ struct StepPlan {
     int tpp;               // 64-cell tiles per z plane
     int tpr;               // row tiles: 64-cell tiles per row (0: the plane tiling)
     bool ahead;            // cell tiles in any_cell's AHEAD form
+    bool aa_rows;          // in-place kernels: row tiles (needs tpr)
     int64_t nblocks_cells; // blocks of 4 wavefronts
     double rxl;            // 1 / xl
     // Two steps per pass (k_bulk2): 64 x 8 cell tiles in x-y, tb_zc planes

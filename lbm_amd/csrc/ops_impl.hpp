@@ -216,7 +216,7 @@ struct OpsImpl {
     template <bool B32>
     static void launch_aa(const StepArgs& a, const StepPlan& p, int phase, hipStream_t s) {
         const dim3 grid(static_cast<uint32_t>(p.nblocks_cells));
-        if (B32 && p.tpr && phase < 2) {
+        if (B32 && p.aa_rows && phase < 2) {
             if (phase == 0)
                 hipLaunchKernelGGL((k_aa_eo<L, M, true, true>), row_grid(a, p), dim3(256), 0, s, a, 0, 0.0, p.tpr);
             else
