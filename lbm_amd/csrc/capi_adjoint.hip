@@ -30,6 +30,7 @@
 #include "dual.hpp"
 #include "lbm_hip.h"
 #include "ops_adjoint.hpp"
+#include "record.hpp"
 
 using namespace lbm_amd;
 
@@ -124,11 +125,9 @@ bool record_run(lbm_tape* t) {
     t->hist_step = static_cast<size_t>(d->L.xl) * d->L.yl * d->L.zl * 4 * t->ops->calc_bytes;
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
-    if (t->T > std::min(total_b / 4, free_b / 2) / t->hist_step) return false;
-    // what the tape allocates beside it: a checkpoint and two mu buffers (where
-    // only those fit, the tape has to fit without a record)
-    const size_t rest = d->field_bytes + 2 * static_cast<size_t>(d->L.plane) * d->Q * t->ops->calc_bytes;
-    if (t->T * t->hist_step + rest > free_b) return false;
+    const size_t rest = tape_rest(d->field_bytes, static_cast<size_t>(d->L.plane), d->Q, t->ops->calc_bytes,
+                                  static_cast<size_t>(d->nb), static_cast<size_t>(d->L.yl) * d->L.zl);
+    if (!record_fits(t->T, t->hist_step, rest, free_b, total_b)) return false;
     if (hipMalloc(&t->hist, t->T * t->hist_step) != hipSuccess) {
         (void)hipGetLastError();
         t->hist = nullptr;

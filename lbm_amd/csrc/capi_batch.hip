@@ -19,6 +19,7 @@
 #include "domain_impl.hpp"
 #include "lbm_hip.h"
 #include "ops_adjoint.hpp"
+#include "record.hpp"
 
 using namespace lbm_amd;
 
@@ -632,8 +633,17 @@ int batch_adj_create(lbm_batch* b, uint64_t nsteps, uint64_t k1, uint64_t k2, bo
     for (const lbm_domain* d : b->doms) record += static_cast<size_t>(stride_of(d)) * cb;
     if (automatic) {
         size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess &&
-            nsteps <= std::min(total_b / 4, free_b / 2) / record && nsteps * record + 3 * field_total <= free_b &&
+        size_t rest = 0;  // three slots per domain, the tables, the gradients
+        size_t elems = 0, near = 0, tiles = 0;
+        for (const lbm_domain* d : b->doms) {
+            rest += allocated(3 * d->field_bytes);
+            elems += static_cast<size_t>(d->L.plane);
+            near += static_cast<size_t>(d->nb);
+            tiles += static_cast<size_t>((static_cast<int64_t>(d->L.xl) * d->L.yl + 63) / 64) * d->L.zl;
+        }
+        rest += allocated(sizeof(int) * elems) + allocated(24 * std::max<size_t>(near, 1)) + allocated(sizeof(TileRef) * tiles) +
+                allocated(sizeof(BatchAdjView) * b->doms.size()) + 2 * allocated(sizeof(double) * 4 * b->doms.size());
+        if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && record_fits(nsteps, record, rest, free_b, total_b) &&
             hipMalloc(&t->hist, nsteps * record) != hipSuccess) {
             (void)hipGetLastError();
             t->hist = nullptr;
