@@ -395,9 +395,11 @@ int lbm_set_index_width(lbm_domain* d, int bits);
  * in-place layout or a vector width set by lbm_set_tuning steps singly.
  * Results on fluid cells are the same bits as single steps. steps_per_pass:
  * 0 (default, automatic): two steps per pass where that measured faster,
- * which leaves domains with boundary cells in 16-bit storage stepping
- * singly, and domains of few cells: under 3 * 2^16 without boundary cells,
- * under 600 000 with, under 3 000 000 with solid cells inside the box;
+ * which leaves stepping singly: domains without boundary cells under 3 * 2^16
+ * cells; with boundary cells, those in 16-bit storage, those whose two buffers
+ * together take more than 32 and at most 256 MiB (the memory-side cache holds
+ * them), those under 600 000 cells, and under 3 000 000 with solid cells inside
+ * the box (lbm_get_steps_per_launch tells);
  * 2: two steps per pass wherever it applies; 1: single steps. z_chunk:
  * planes per block of the pass (0 = automatic). No reference counterpart: a scheduling
  * choice of this implementation. */

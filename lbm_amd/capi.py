@@ -323,10 +323,11 @@ class Domain:
         _check(load().lbm_set_index_width(self._h, bits))
 
     def set_time_blocking(self, steps_per_pass: int = 0, z_chunk: int = 0) -> None:
-        """0 (default): two steps per pass where that measured faster
-        (bulk-only domains in fp32/fp16/bf16; fp32 D3Q15/D3Q19 domains with
-        boundary cells); 2: two steps per pass wherever it applies (also fp32
-        D3Q27 domains with boundary cells); 1: single steps."""
+        """0 (default): two steps per pass where that measured faster (bulk-only
+        domains in fp32/fp16/bf16 and fp32 domains with boundary cells, from the
+        sizes that include/lbm_hip.h names); 2: two steps per pass wherever it
+        applies (also 16-bit domains with boundary cells); 1: single steps.
+        info()["steps_per_launch"] tells which."""
         _check(load().lbm_set_time_blocking(self._h, steps_per_pass, z_chunk))
 
 

@@ -224,14 +224,22 @@ int make_plan(lbm_domain* d) {
     // and with walls the emit launch before it. With walls the pass also holds
     // half as many wavefronts as the cell tiles, and where solid cells idle
     // its lanes and put surfaces into most tiles it pays only on fields well
-    // beyond the caches. Measured, us per step, single / pass, fp32:
+    // beyond the caches. Measured, us per step, single / pass, fp32 (MiB of
+    // both buffers):
     //   periodic D3Q19: 48^3 6.7 / 7.8, 64^3 8.9 / 9.1, 96^3 32.3 / 20.5
     //     (D3Q15, D3Q27 and 16-bit storage cross at the same sizes);
-    //   cavity D3Q19: 64^3 16.4 / 18.4, 80^3 26.4 / 30.9, 96^3 36.5 / 32.8,
-    //     192^3 207 / 156; D3Q27: 96^3 50.1 / 52.4, 128^3 94.8 / 81.7;
-    //   channel around spheres (fluid 0.8): D3Q19 192x96x96 60.5 / 72.7,
-    //     256x128x128 171 / 148; D3Q27 91.7 / 120, 258 / 243;
-    //   pipe 208x100x100: D3Q19 63.1 / 86.0, D3Q27 90.9 / 153.
+    //   cavity D3Q19: 64^3 (61) 11.5 / 17.2, 96^3 (178) 25.8 / 31.1, 112^3
+    //     (241) 45.3 / 45.2, 116^3 (258) 62.4 / 47.8, 192^3 205 / 154;
+    //     D3Q15: 120^3 (218) 39.3 / 42.8, 128^3 (309) 49.9 / 47.2, 160^3 93.2 /
+    //     96.2; D3Q27: 96^3 (253) 36.1 / 50.0, 104^3 (296) 58.7 / 59.7, 128^3
+    //     89.0 / 80.1, 160^3 165 / 166;
+    //   channel around spheres (fluid 0.8), 1.8, 3.4 and 6.2 million cells:
+    //     D3Q19 60.9 / 68.4, 123 / 123, 240 / 221; D3Q27 88.7 / 111, 184 / 198,
+    //     350 / 400 (14 million: 796 / 735);
+    //   pipe, 2.1, 6.2 and 33 million cells: D3Q19 58.2 / 83.1, 157 / 203, 787 /
+    //     755; D3Q27 83.9 / 147, 224 / 363, 1154 / 1276.
+    // (With walls alone the size of the buffers decides; the 600 000 cells only
+    // keep what takes at most 32 MiB single.)
     const int64_t least = !walled ? 3 * 65536 : (d->n_fluid == static_cast<uint64_t>(cells) ? 600000 : 3000000);
     // With walls the cell tiles also gain more from output kept in the
     // memory-side cache (Put::Keep) than the pass does.
