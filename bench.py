@@ -18,16 +18,16 @@ OpenMP on the host cores, bounded sample).
 Further legs ride on the same line:
 - "walled": the 256^3 lid-driven cavity (D3Q19, tau 0.6) and a 384x192x192
   channel around seeded spheres (D3Q27, tau 0.55), fp32 and fp16, each as
-  two steps per pass (k_wall2) and as single steps (k_cells), with the form
+  two steps per pass (k_wall2) and as single steps (k_cell_rows), with the form
   lbm_step picks by default named;
 - "report": the periodic box in fp64 (the reference's operation order) and
   in D3Q15 / D3Q27;
 - "inplace_aa": the same workload in the in-place (AA) layout, one buffer;
 - "adjoint": the inverse problem on a periodic 128^3 D3Q19 fp32 box with a
   Brinkman porosity field (seeded uniform 32^3, trilinear), body force 1e-5 x,
-  2000 steps with sqrt(N) checkpoints, plane-velocity misfit objective: wall
-  time of the forward pass, of the checkpoint recompute and of the adjoint
-  sweep, and their ratio;
+  2000 steps, recorded where the record fits in device memory and with sqrt(N)
+  checkpoints else, plane-velocity misfit objective: wall time of the forward
+  pass, of the checkpoint recompute and of the adjoint sweep, and their ratio;
 - "batch": 512 lid-driven D3Q19 fp32 cavities (edges log-uniform in
   [16, 96], Re uniform in [10, 1000] through per-domain tau) stepped 2000
   times in one graph-captured launch per step after autotuning, then the
@@ -74,7 +74,7 @@ def tgv(n: int, seed: int = 12345):
 
 def traffic_from_profiles(mode: str, kernel: str = "bulk", workload: str = "d3q19_256"):
     """HBM bytes per launch of a kernel (bulk: k_bulk, pass: k_bulk2, cells:
-    k_cells) on a workload, measured by rocprofv3 --pmc (FETCH_SIZE +
+    k_cell_rows) on a workload, measured by rocprofv3 --pmc (FETCH_SIZE +
     WRITE_SIZE, each scaled by the copy-kernel calibration), from the
     committed summary profiles/pmc_<kernel>_<workload>_<mode>.txt; None when
     absent."""
@@ -138,7 +138,7 @@ def mode_row(r: dict, mode: str, q: int = Q) -> dict:
 
 def walled_case(capi, name: str, q: int, mode: str, dims, tau: float, sc, steps: int, warmup: int = 5):
     """One walled workload, as two steps per pass (k_wall2, forced where the
-    domain allows it) and as single steps (64-cell tiles, k_cells), with the
+    domain allows it) and as single steps (64-cell tiles, k_cell_rows), with the
     form lbm_step picks by default named: event-timed kernel time per
     launch, MLUPS over interior and
     over fluid cells, and the roofline on the bytes a launch must move (each
@@ -164,7 +164,7 @@ def walled_case(capi, name: str, q: int, mode: str, dims, tau: float, sc, steps:
         interior, fluid = info["ncells_interior"], info["ncells_fluid"]
         moved = 2 * q * BYTES[mode] * fluid
         gbs = moved / (kernel_ms * 1e-3) / 1e9
-        kname = "k_wall2" if k == 2 else ("k_cells" if info["cell_tiles"] else "k_bulk+k_near")
+        kname = "k_wall2" if k == 2 else ("k_cell_rows" if info["cell_tiles"] else "k_bulk+k_near")
         traffic = traffic_from_profiles(mode, "wall2" if k == 2 else "cells", name)
         row = {"kernel": kname, "steps_per_launch": k, "kernel_ms": round(kernel_ms, 5),
                "ms_per_step": round(ev["total_ms"] / steps, 5),
@@ -299,7 +299,7 @@ def adjoint_leg(capi, steps: int = 2000):
     d.close()
     fwd = tm["forward_ms"]
     return {"workload": "D3Q19 periodic 128^3 Brinkman, g=1e-5 x, tau=0.8, fp32, plane-misfit objective",
-            "steps": steps, "checkpoints": "sqrt(N)",
+            "steps": steps, "checkpoints": "sqrt(N)" if tm["recompute_ms"] > 0.1 else "none (recorded forward run)",
             "forward_ms": round(fwd, 3), "recompute_ms": round(tm["recompute_ms"], 3),
             "adjoint_ms": round(tm["adjoint_ms"], 3),
             "adjoint_step_over_forward_step": round(tm["adjoint_ms"] / fwd, 3),

@@ -114,11 +114,13 @@ struct StepArgs {
     double g[3];
     // Kernels built with HIST: 4 Calc values (drho, u) of the incoming
     // populations per interior cell, x fastest, written here by the step (and
-    // by a two-step pass's second step at hist2). Written and read past the
-    // caches: each value is used once, a whole sweep later, and displaced lines
-    // that the step itself reads again (objective and gradient, plain / non-
-    // temporal: 128^3 porosity, 100 steps 11.8 / 11.5 ms; 64 mixed cavities, 50
-    // steps 30.4 / 29.6 ms).
+    // by a two-step pass's second step at hist2). The two-step passes and the
+    // batched steps write and read it past the caches (k_adj2 its step t - 1
+    // only: ring cells take step t's from several blocks): each value is used
+    // once, a whole sweep later, and displaced lines that the step itself reads
+    // again (objective and gradient, plain / non-temporal: 128^3 porosity, 100
+    // steps 11.8 / 11.5 ms; 64 mixed cavities, 50 steps 30.4 / 29.6 ms). The
+    // single steps of the row kernel and k_adj_hist access it plainly.
     void* hist;
     void* hist2;
     // any_cell built with HIST: index of a NEAR cell in the domain's list per
